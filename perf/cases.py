@@ -16,9 +16,9 @@ repository's kernels.
 Weights are random with a trained model's scales: projections N(0, 0.02) (the
 quantized ones as the codes and group scales such a matrix has), norm weights
 log-uniform in [0.5, 2] (what the AWQ fold leaves), embeddings scaled so that
-the logits have a standard deviation of about 3, which gives distributions as
-peaked as a language model's and drafts that agree with their target part of
-the time.
+the logits have a standard deviation of about 3, which gives distributions
+about as peaked as a language model's. Two such models seldom agree, so a
+speculative step emits one token; its device work does not depend on that.
 """
 from __future__ import annotations
 
