@@ -1261,8 +1261,13 @@ int fg_kv_create(fg_ctx* ctx, int32_t layers, int32_t kv_heads, int32_t head_dim
         fg_kv_destroy(kv);
         return fail(FG_E_NOMEM, "cache allocation failed");
     }
-    HIPCHK(hipMemset(kv->k, 0, bytes));
-    HIPCHK(hipMemset(kv->v, 0, bytes));
+    // cleared on the context's stream: it does not wait for the default stream, so a
+    // clear queued there could still be running over the first rows written here
+    if (hipMemsetAsync(kv->k, 0, bytes, ctx->stream) != hipSuccess ||
+        hipMemsetAsync(kv->v, 0, bytes, ctx->stream) != hipSuccess) {
+        fg_kv_destroy(kv);
+        return fail(FG_E_DEVICE, "cache clear failed");
+    }
     *out = kv;
     return 0;
 }
