@@ -1387,7 +1387,7 @@ int fg_forward_capture(fg_ctx* ctx, const fg_model* m, fg_kv* kv, const fg_chunk
 // Distributions of rows carved from the context's sampling buffer starting at
 // row `first` (the buffer holds `total` rows of `cap` pairs): tok, pr, tok_id,
 // pr_id [total][cap], n [total]; with wide rows also dense [total][cap] and
-// the sort scratch [total][4 cap].
+// the sort scratch [total][wide_scratch_words(cap)].
 static size_t sample_cap(bool wide, int vocab) { return wide ? (size_t)vocab : (size_t)kSampleCap; }
 static SampleRows sample_rows(void* buf, int total, int first, bool wide, int vocab) {
     const size_t cap = sample_cap(wide, vocab), tc = (size_t)total * cap;
@@ -1402,12 +1402,12 @@ static SampleRows sample_rows(void* buf, int total, int first, bool wide, int vo
     r.cap = (int)cap;
     r.vocab = vocab;
     r.dense = wide ? (float*)(b + o_dense) + (size_t)first * cap : nullptr;
-    r.scratch = wide ? (uint32_t*)(b + o_dense + tc * 4) + (size_t)first * cap * 4 : nullptr;
+    r.scratch = wide ? (uint32_t*)(b + o_dense + tc * 4) + (size_t)first * wide_scratch_words((int)cap) : nullptr;
     return r;
 }
 static size_t sample_bytes(int total, bool wide, int vocab) {
     const size_t tc = (size_t)total * sample_cap(wide, vocab);
-    return tc * 16 + ((size_t)total * 4 + 255) / 256 * 256 + (wide ? tc * 20 : 0);
+    return tc * 16 + ((size_t)total * 4 + 255) / 256 * 256 + (wide ? tc * 4 + (size_t)total * wide_scratch_words(vocab) * 4 : 0);
 }
 static_assert(sizeof(SampleParams) == sizeof(fg_sampling), "fg_sampling is copied to the device as SampleParams");
 

@@ -279,8 +279,13 @@ struct SampleRows {
     int cap;    // pairs per row: kSampleCap, or the vocabulary when any row is wide
     int vocab;
     float* dense;        // wide rows: probability by token [row][cap] (null: no wide rows)
-    uint32_t* scratch;   // wide rows: the sort's ping-pong keys and values [row][4 * cap]
+    uint32_t* scratch;   // wide rows: the sort's buffers [row][wide_scratch_words(cap)] (null: no wide rows)
 };
+// Words of scratch of a wide row: two keys and two tokens per entry, four passes of 256 digit
+// counts per 1024 entries, and 64 words for its sums.
+__host__ __device__ inline size_t wide_scratch_words(int cap) {
+    return 4 * (size_t)cap + 1024 * (((size_t)cap + 1023) / 1024) + 64;
+}
 // A row is wide when it samples with top_k 0 (no limit) or above kSampleCap.
 __host__ __device__ inline bool sample_wide(const SampleParams& p) {
     return p.temperature > 0.0f && (p.top_k == 0 || p.top_k > kSampleCap);

@@ -10,9 +10,9 @@
 // lookups and the residual, which the reference builds in token order). A
 // wide one (top_k 0, no limit, or above kSampleCap) keeps up to the whole
 // vocabulary in the reference's order plus a dense by-token copy; its kernels
-// (k_dist_wide, k_draw_wide, k_accept_wide) run after the small ones, each
+// (k_wide_*, k_draw_wide, k_accept_wide) run after the small ones, each
 // kind skipping the other's rows.
-#include "internal.h"
+#include "seqsum.h"
 
 #include <math.h>
 
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(kSampleCap) void k_dist(const float* __restrict__ l
         if (tid == 0) n_out[row] = 0;
         return;
     }
-    if (sample_wide(p)) return;  // k_dist_wide
+    if (sample_wide(p)) return;  // k_wide_*
     const float* lg = logits + (size_t)row * vocab;
     const float t = p.temperature > 1e-5f ? p.temperature : 1e-5f;
     const int K = min(p.top_k, vocab);
@@ -339,223 +339,228 @@ __global__ void k_accept_sampled(int n_seqs, int k, const SampleParams* __restri
 // Wide distributions: top_k = 0 (no limit) or above kSampleCap. A row holds up
 // to `cap` (the vocabulary) pairs, in the reference's order, plus a dense
 // token-indexed copy of the probabilities (0 where a token is not kept) for
-// the acceptance's lookups and residual. One workgroup per row or sequence.
-// The reference's sums and walks are sequential (f64 softmax sum, f32 top-p
-// prefix, f32 draw sums): one thread runs them in order over values the
-// whole workgroup stages in LDS, BATCH at a time.
+// the acceptance's lookups and residual. The work over the vocabulary runs on
+// one workgroup per 1024 tokens and row: the keys, a stable LSD radix sort
+// (four 8-bit passes), the exponentials and the final probabilities. The
+// reference's sums and walks are sequential (f64 softmax sum, f32 top-p
+// prefix, f32 draw sums); one workgroup per row or sequence runs them with
+// seq_scan, which has the sequential loop's bits.
+// Bound: the latency of eight dependent launches. 49,152 tokens, 4 rows: 2664
+// us for the whole distribution on one workgroup a row (its tiles of the sort
+// one after the other, its sums one lane each), 8008 us for the acceptance;
+// now 145 us (sort 4 x 14, sums 71) and 191 us.
 // ---------------------------------------------------------------------------
-constexpr int kWideThreads = 1024;
+constexpr int kWideTile = 1024;  // tokens per workgroup
 
-// Stable LSD radix sort of n (key, value) pairs, ascending by key, four 8-bit
-// passes through global ping-pong buffers (k0/v0 -> k1/v1 -> k0/v0 ...; the
-// result ends in k0/v0). Each 1024-element tile ranks its elements by digit
-// with wave ballots (equal digits keep element order), then scatters after
-// the digit's running offset.
-__device__ void radix_sort_wide(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, int n) {
+// A wide row's scratch: keys and tokens (two of each, the sort's ping-pong), the four passes'
+// digit counts [pass][tile][256], and the softmax sum, the top-p sum and whether it applies.
+struct WideRow {
+    uint32_t *k0, *v0, *k1, *v1, *hist;
+    double* dsum;
+    float* s2;
+    int* cut;
+};
+__device__ __forceinline__ WideRow wide_row(const SampleRows& d, int row) {
+    uint32_t* p = d.scratch + (size_t)row * wide_scratch_words(d.cap);
+    WideRow w;
+    w.k0 = p;
+    w.v0 = p + d.cap;
+    w.k1 = p + 2 * (size_t)d.cap;
+    w.v1 = p + 3 * (size_t)d.cap;
+    w.hist = p + 4 * (size_t)d.cap;
+    uint32_t* t = p + wide_scratch_words(d.cap) - 64;
+    w.dsum = (double*)t;
+    w.s2 = (float*)(t + 2);
+    w.cut = (int*)(t + 3);
+    return w;
+}
+
+// The complemented keys of a tile (ascending: value descending), its tokens, the first pass's
+// digit counts; the later passes' counts and the dense copy cleared.
+__global__ __launch_bounds__(kWideTile) void k_wide_keys(const float* __restrict__ logits, int vocab, int rows_per_seq,
+                                                         const SampleParams* __restrict__ prm, SampleRows d) {
     __shared__ uint32_t hist[256];
-    __shared__ uint32_t wcnt[kWideThreads / 64][256];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint64_t below = (1ull << lane) - 1;
-    for (int i = tid; i < (kWideThreads / 64) * 256; i += kWideThreads) (&wcnt[0][0])[i] = 0;
-    for (int pass = 0; pass < 4; pass++) {
-        const int shift = 8 * pass;
-        if (tid < 256) hist[tid] = 0;
-        __syncthreads();
-        for (int i = tid; i < n; i += kWideThreads) atomicAdd(&hist[(k0[i] >> shift) & 255u], 1u);
-        __syncthreads();
-        if (tid == 0) {
-            uint32_t run = 0;
-            for (int d = 0; d < 256; d++) {
-                const uint32_t c = hist[d];
-                hist[d] = run;
-                run += c;
-            }
-        }
-        __syncthreads();
-        for (int t0 = 0; t0 < n; t0 += kWideThreads) {
-            const int i = t0 + tid;
-            const bool valid = i < n;
-            const uint32_t key = valid ? k0[i] : 0u, val = valid ? v0[i] : 0u;
-            const uint32_t d = (key >> shift) & 255u;
-            uint64_t m = __ballot(valid);
-#pragma unroll
-            for (int b = 0; b < 8; b++) {
-                const uint64_t bb = __ballot((d >> b) & 1u);
-                m &= ((d >> b) & 1u) ? bb : ~bb;
-            }
-            const int rank = __popcll(m & below);
-            if (valid && rank == 0) wcnt[wave][d] = __popcll(m);
-            __syncthreads();
-            if (tid < 256) {
-                uint32_t run = hist[tid];
-                for (int w = 0; w < kWideThreads / 64; w++) {
-                    const uint32_t c = wcnt[w][tid];
-                    wcnt[w][tid] = run;
-                    run += c;
-                }
-                hist[tid] = run;
-            }
-            __syncthreads();
-            if (valid) {
-                const uint32_t dst = wcnt[wave][d] + rank;
-                k1[dst] = key;
-                v1[dst] = val;
-            }
-            __syncthreads();
-            for (int z = tid; z < (kWideThreads / 64) * 256; z += kWideThreads) (&wcnt[0][0])[z] = 0;
-            __syncthreads();
-        }
-        uint32_t* tk = k0;
-        k0 = k1;
-        k1 = tk;
-        uint32_t* tv = v0;
-        v0 = v1;
-        v1 = tv;
-    }
-}
-
-// Thread 0 visits v(i) for i = 0, 1, ... < n in order: the workgroup stages
-// BATCH values at a time in LDS (`stage`); visit(i, value) returns true to
-// stop. Every thread of the workgroup must call it.
-template <int BATCH, class Value, class Visit>
-__device__ void ordered_scan(int n, float* stage, Value value, Visit visit) {
-    __shared__ int stop;
-    if (threadIdx.x == 0) stop = 0;
-    for (int i0 = 0; i0 < n; i0 += BATCH) {
-        __syncthreads();
-        for (int i = threadIdx.x; i < BATCH; i += blockDim.x) stage[i] = i0 + i < n ? value(i0 + i) : 0.0f;
-        __syncthreads();
-        if (threadIdx.x == 0)
-            for (int i = 0; i < BATCH && i0 + i < n; i++)
-                if (visit(i0 + i, stage[i])) {
-                    stop = 1;
-                    break;
-                }
-        __syncthreads();
-        if (stop) break;
-    }
-    __syncthreads();
-}
-
-// sampler::distribution for rows whose top_k is 0 or above kSampleCap (other
-// rows are k_dist's): the keys sorted by value descending and token ascending
-// (a stable ascending sort of the complemented keys in token order), exp(v -
-// max) for the top K, their f64 sum in that order, probabilities, the top-p
-// prefix; the pairs in that order (tok, pr) and the dense copy.
-__global__ __launch_bounds__(kWideThreads) void k_dist_wide(const float* __restrict__ logits, int vocab,
-                                                            int rows_per_seq, const SampleParams* __restrict__ prm,
-                                                            SampleRows d) {
-    __shared__ float stage[kWideThreads];
-    __shared__ double dsum_s;
-    __shared__ int keep_s;
-    __shared__ float s2_s;
-    const int row = blockIdx.x, tid = threadIdx.x;
+    const int row = blockIdx.y, tid = threadIdx.x, i = blockIdx.x * kWideTile + tid, tiles = gridDim.x;
     const SampleParams p = prm[row / rows_per_seq];
     if (!sample_wide(p)) return;  // greedy rows and small top_k rows: k_dist
-    const size_t base = (size_t)row * d.cap;
-    const float* lg = logits + (size_t)row * vocab;
+    const WideRow w = wide_row(d, row);
     const float t = p.temperature > 1e-5f ? p.temperature : 1e-5f;
-    const int K = p.top_k == 0 ? vocab : min(p.top_k, vocab);
-    uint32_t* k0 = d.scratch + (size_t)row * d.cap * 4;
-    uint32_t *v0 = k0 + d.cap, *k1 = v0 + d.cap, *v1 = k1 + d.cap;
-    for (int i = tid; i < vocab; i += kWideThreads) {
-        k0[i] = ~total_key(lg[i] / t);
-        v0[i] = (uint32_t)i;
+    if (tid < 256) hist[tid] = 0;
+    __syncthreads();
+    if (i < vocab) {
+        const uint32_t key = ~total_key(logits[(size_t)row * vocab + i] / t);
+        w.k0[i] = key;
+        w.v0[i] = (uint32_t)i;
+        d.dense[(size_t)row * d.cap + i] = 0.0f;
+        atomicAdd(&hist[key & 255u], 1u);
     }
     __syncthreads();
-    radix_sort_wide(k0, v0, k1, v1, vocab);
-    float* pr = d.pr + base;
-    uint32_t* tok = d.tok + base;
-    const float mx = key_value(~k0[0]);
-    for (int i = tid; i < K; i += kWideThreads) pr[i] = expf_rounded(key_value(~k0[i]) - mx);
-    __syncthreads();
-    // the f64 sum in the reference's order
-    {
-        double sum = 0.0;
-        ordered_scan<kWideThreads>(K, stage, [&](int i) { return pr[i]; }, [&](int, float e) {
-            sum += (double)e;
-            return false;
-        });
-        if (tid == 0) dsum_s = sum;
-        __syncthreads();
+    if (tid < 256) {
+        w.hist[(size_t)blockIdx.x * 256 + tid] = hist[tid];
+#pragma unroll
+        for (int pass = 1; pass < 4; pass++) w.hist[((size_t)pass * tiles + blockIdx.x) * 256 + tid] = 0;
     }
-    const double dsum = dsum_s;
-    for (int i = tid; i < K; i += kWideThreads) pr[i] = (float)((double)pr[i] / dsum);
-    __syncthreads();
-    int n = K;
-    if (p.top_p < 1.0f) {
-        int keep = K;
-        float acc = 0.0f;
-        ordered_scan<kWideThreads>(K, stage, [&](int i) { return pr[i]; }, [&](int i, float v) {
-            acc += v;
-            if (acc >= p.top_p) {
-                keep = i + 1;
-                return true;
-            }
-            return false;
-        });
-        if (tid == 0) keep_s = keep;
-        __syncthreads();
-        n = keep_s;
-        float s2 = 0.0f;
-        ordered_scan<kWideThreads>(n, stage, [&](int i) { return pr[i]; }, [&](int, float v) {
-            s2 += v;
-            return false;
-        });
-        if (tid == 0) s2_s = s2;
-        __syncthreads();
-        const float ss = s2_s;
-        for (int i = tid; i < n; i += kWideThreads) pr[i] = pr[i] / ss;
-    }
-    float* dense = d.dense + base;
-    for (int i = tid; i < vocab; i += kWideThreads) dense[i] = 0.0f;
-    __syncthreads();
-    for (int i = tid; i < n; i += kWideThreads) {
-        tok[i] = v0[i];
-        dense[v0[i]] = pr[i];
-    }
-    if (tid == 0) d.n[row] = n;
 }
 
-// sampler::draw over a wide row's n pairs, on the workgroup; thread 0 holds
-// the generator. Returns the token on thread 0.
-__device__ uint32_t draw_wide(const uint32_t* tok, const float* pr, int n, uint64_t& rng, float* stage) {
-    float s = 0.0f;
-    ordered_scan<256>(n, stage, [&](int i) { return pr[i]; }, [&](int, float v) {
-        s += v;
-        return false;
-    });
-    uint32_t out = n > 0 ? tok[n - 1] : 0;
-    if (threadIdx.x == 0) {
-        float u = (float)rng_uniform(rng) * s;
-        // the walk: thread 0 keeps u; staged like the sum
-        stage[256] = u;
-    }
-    float u = 0.0f;
-    if (threadIdx.x == 0) u = stage[256];
-    ordered_scan<256>(n, stage, [&](int i) { return pr[i]; }, [&](int i, float v) {
-        if (u < v) {
-            out = tok[i];
-            return true;
+// One 8-bit pass of the stable LSD radix sort, one workgroup per tile of 1024: a digit's place is
+// the count of smaller digits, plus its count in earlier tiles, plus its rank in the tile (wave
+// ballots keep element order). The elements are counted for the next pass where they land.
+__global__ __launch_bounds__(kWideTile) void k_wide_sort(int vocab, int pass, int rows_per_seq,
+                                                         const SampleParams* __restrict__ prm, SampleRows d) {
+    __shared__ uint32_t tot[4][256], bel[4][256], wsum[4];
+    __shared__ uint32_t wcnt[kWideTile / 64][256];
+    const int row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, tiles = gridDim.x;
+    if (!sample_wide(prm[row / rows_per_seq])) return;
+    const WideRow w = wide_row(d, row);
+    const uint32_t *ki = pass & 1 ? w.k1 : w.k0, *vi = pass & 1 ? w.v1 : w.v0;
+    uint32_t *ko = pass & 1 ? w.k0 : w.k1, *vo = pass & 1 ? w.v0 : w.v1;
+    const uint32_t* hist = w.hist + (size_t)pass * tiles * 256;
+    const int i = blockIdx.x * kWideTile + tid, shift = 8 * pass;
+    const bool valid = i < vocab;
+    const uint32_t key = valid ? ki[i] : 0u, val = valid ? vi[i] : 0u;
+#pragma unroll
+    for (int z = 0; z < 4; z++) (&wcnt[0][0])[z * kWideTile + tid] = 0;
+    {
+        // each quarter of the workgroup sums a quarter of the tiles' counts
+        const int dg = tid & 255, part = tid >> 8;
+        uint32_t all = 0, below = 0;
+#pragma unroll 8
+        for (int t = part; t < tiles; t += 4) {
+            const uint32_t c = hist[(size_t)t * 256 + dg];
+            all += c;
+            below += t < (int)blockIdx.x ? c : 0u;
         }
-        u -= v;
-        return false;
-    });
-    return out;
+        tot[part][dg] = all;
+        bel[part][dg] = below;
+    }
+    __syncthreads();
+    uint32_t excl = 0, mine = 0;
+    if (tid < 256) {
+        mine = tot[0][tid] + tot[1][tid] + tot[2][tid] + tot[3][tid];
+        uint32_t inc = mine;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t v = __shfl_up(inc, o, 64);
+            if (lane >= o) inc += v;
+        }
+        if (lane == 63) wsum[wave] = inc;
+        excl = inc - mine;
+    }
+    // this tile's ranks meanwhile
+    const uint32_t dgt = (key >> shift) & 255u;
+    uint64_t same = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < 8; b++) {
+        const uint64_t bb = __ballot((dgt >> b) & 1u);
+        same &= ((dgt >> b) & 1u) ? bb : ~bb;
+    }
+    const int rank = __popcll(same & ((1ull << lane) - 1));
+    if (valid && rank == 0) wcnt[wave][dgt] = __popcll(same);
+    __syncthreads();
+    if (tid < 256) {
+        uint32_t run = excl + bel[0][tid] + bel[1][tid] + bel[2][tid] + bel[3][tid];
+        for (int v = 0; v < wave; v++) run += wsum[v];
+#pragma unroll
+        for (int v = 0; v < kWideTile / 64; v++) {
+            const uint32_t c = wcnt[v][tid];
+            wcnt[v][tid] = run;
+            run += c;
+        }
+    }
+    __syncthreads();
+    if (valid) {
+        const uint32_t dst = wcnt[wave][dgt] + rank;
+        ko[dst] = key;
+        vo[dst] = val;
+        if (pass < 3)
+            atomicAdd(&w.hist[((size_t)(pass + 1) * tiles + dst / kWideTile) * 256 + ((key >> (shift + 8)) & 255u)], 1u);
+    }
+}
+
+// exp(v - max) of the sorted row's first K values
+__global__ __launch_bounds__(kWideTile) void k_wide_exp(int vocab, int rows_per_seq,
+                                                        const SampleParams* __restrict__ prm, SampleRows d) {
+    const int row = blockIdx.y, i = blockIdx.x * kWideTile + threadIdx.x;
+    const SampleParams p = prm[row / rows_per_seq];
+    if (!sample_wide(p)) return;
+    const WideRow w = wide_row(d, row);
+    const int K = p.top_k == 0 ? vocab : min(p.top_k, vocab);
+    if (i < K) d.pr[(size_t)row * d.cap + i] = expf_rounded(key_value(~w.k0[i]) - key_value(~w.k0[0]));
+}
+
+// The f64 sum of a row's exponentials and its top-p prefix. The reference then sums the kept
+// probabilities again from the start: the prefix's own sum.
+__global__ __launch_bounds__(1024) void k_wide_sums(int vocab, int rows_per_seq, const SampleParams* __restrict__ prm,
+                                                    SampleRows d) {
+    __shared__ SeqShared<double> sd;
+    __shared__ SeqShared<float> sf;
+    const int row = blockIdx.x;
+    const SampleParams p = prm[row / rows_per_seq];
+    if (!sample_wide(p)) return;
+    const WideRow w = wide_row(d, row);
+    const int K = p.top_k == 0 ? vocab : min(p.top_k, vocab);
+    const float* e = d.pr + (size_t)row * d.cap;
+    double sum = 0.0;
+    seq_scan<SEQ_SUM, 8, double>(K, sum, 0.0, [&](int i) { return e[i]; }, sd);
+    int n = K;
+    float acc = 0.0f;
+    const bool cut = p.top_p < 1.0f;
+    if (cut) {
+        auto prob = [&](int i) { return (float)((double)e[i] / sum); };
+        if (p.top_p > 0.0f) {
+            const int at = seq_scan<SEQ_REACH, 4, float>(K, acc, p.top_p, prob, sf);
+            n = at < K ? at + 1 : K;
+        } else {
+            acc = prob(0);
+            if (acc >= p.top_p) n = 1;  // (a NaN reaches no limit, and stays one)
+        }
+    }
+    if (threadIdx.x == 0) {
+        *w.dsum = sum;
+        *w.s2 = acc;
+        *w.cut = cut;
+        d.n[row] = n;
+    }
+}
+
+// The kept pairs in the reference's order and the dense copy
+__global__ __launch_bounds__(kWideTile) void k_wide_pairs(int rows_per_seq, const SampleParams* __restrict__ prm,
+                                                          SampleRows d) {
+    const int row = blockIdx.y, i = blockIdx.x * kWideTile + threadIdx.x;
+    if (!sample_wide(prm[row / rows_per_seq]) || i >= d.n[row]) return;
+    const WideRow w = wide_row(d, row);
+    const size_t at = (size_t)row * d.cap;
+    float v = (float)((double)d.pr[at + i] / *w.dsum);
+    if (*w.cut) v = v / *w.s2;
+    const uint32_t t = w.v0[i];
+    d.pr[at + i] = v;
+    d.tok[at + i] = t;
+    d.dense[at + t] = v;
+}
+
+// sampler::draw over a wide row's n pairs, on the workgroup; every thread ends with the token
+// and the advanced generator.
+__device__ uint32_t draw_wide(const uint32_t* tok, const float* pr, int n, uint64_t& rng, SeqShared<float>& sh) {
+    auto value = [&](int i) { return pr[i]; };
+    float s = 0.0f;
+    seq_scan<SEQ_SUM, 4, float>(n, s, 0.0f, value, sh);
+    float u = (float)rng_uniform(rng) * s;
+    const int at = seq_scan<SEQ_WALK, 4, float>(n, u, 0.0f, value, sh);
+    return n > 0 ? tok[min(at, n - 1)] : 0;
 }
 
 // One workgroup per row: sampler::sample of each wide sampled row into
 // out[row * out_stride + out_off].
-__global__ __launch_bounds__(256) void k_draw_wide(int rows, const SampleParams* __restrict__ prm, SampleRows d,
-                                                   uint64_t* __restrict__ rng, uint32_t* __restrict__ out,
-                                                   int out_stride, int out_off) {
-    __shared__ float stage[257];
+__global__ __launch_bounds__(1024) void k_draw_wide(int rows, const SampleParams* __restrict__ prm, SampleRows d,
+                                                    uint64_t* __restrict__ rng, uint32_t* __restrict__ out,
+                                                    int out_stride, int out_off) {
+    __shared__ SeqShared<float> sh;
     const int r = blockIdx.x;
     const SampleParams p = prm[r];
     if (!sample_wide(p)) return;
     uint64_t s = rng[r];
     const size_t base = (size_t)r * d.cap;
-    const uint32_t t = draw_wide(d.tok + base, d.pr + base, d.n[r], s, stage);
+    const uint32_t t = draw_wide(d.tok + base, d.pr + base, d.n[r], s, sh);
     if (threadIdx.x == 0) {
         out[(size_t)r * out_stride + out_off] = t;
         rng[r] = s;
@@ -564,15 +569,15 @@ __global__ __launch_bounds__(256) void k_draw_wide(int rows, const SampleParams*
 
 // One workgroup per sequence: k_accept_sampled's rule for sequences whose
 // distributions are wide (dense lookups; the residual max(0, p - q) and the
-// dense pairs of p in token order over the whole vocabulary).
-__global__ __launch_bounds__(256) void k_accept_wide(int n_seqs, int k, int vocab, const SampleParams* __restrict__ prm,
-                                                     const uint32_t* __restrict__ vtok,
-                                                     const uint32_t* __restrict__ am, SampleRows p, SampleRows q,
-                                                     uint64_t* __restrict__ rng, uint32_t* __restrict__ out_tokens,
-                                                     int32_t* __restrict__ out_count,
-                                                     int32_t* __restrict__ out_accepted) {
-    __shared__ float stage[257];
-    __shared__ int take_s;
+// dense pairs of p in token order over the whole vocabulary). Every thread
+// follows the same generator.
+__global__ __launch_bounds__(1024) void k_accept_wide(int n_seqs, int k, int vocab, const SampleParams* __restrict__ prm,
+                                                      const uint32_t* __restrict__ vtok,
+                                                      const uint32_t* __restrict__ am, SampleRows p, SampleRows q,
+                                                      uint64_t* __restrict__ rng, uint32_t* __restrict__ out_tokens,
+                                                      int32_t* __restrict__ out_count,
+                                                      int32_t* __restrict__ out_accepted) {
+    __shared__ SeqShared<float> sh;
     const int sq = blockIdx.x;
     const SampleParams pp = prm[sq];
     if (!sample_wide(pp)) return;
@@ -580,69 +585,43 @@ __global__ __launch_bounds__(256) void k_accept_wide(int n_seqs, int k, int voca
     uint64_t st = rng[sq];
     int ne = 0, accepted = 0;
     uint32_t* out = out_tokens + (size_t)sq * K1;
+    // a draw from the terms in token order: u walks them down; the token whose term exceeds what
+    // is left of u, or the last token with a positive term (0 when there is none)
+    auto draw = [&](auto term) -> uint32_t {
+        float s = 0.0f;
+        seq_scan<SEQ_SUM, 4, float>(vocab, s, 0.0f, term, sh);
+        float u = (float)rng_uniform(st) * s;
+        const int at = seq_scan<SEQ_WALK, 4, float>(vocab, u, 0.0f, term, sh);
+        if (at < vocab) return (uint32_t)at;
+        __syncthreads();
+        if (threadIdx.x == 0) sh.start = 0;
+        __syncthreads();
+        for (int i = threadIdx.x; i < vocab; i += blockDim.x)
+            if (term(i) > 0.0f) atomicMax(&sh.start, i);
+        __syncthreads();
+        return (uint32_t)sh.start;
+    };
     for (int j = 0; j < k; j++) {
         const int row = sq * K1 + j;
         const uint32_t dtok = vtok[(size_t)sq * K1 + 1 + j];
         const float* pd = p.dense + (size_t)row * p.cap;
         const float* qd = q.dense + ((size_t)j * n_seqs + sq) * q.cap;
-        if (threadIdx.x == 0) {
-            const float px = pd[dtok], qx = qd[dtok];
-            take_s = qx > 0.0f && rng_uniform(st) < (double)fminf(px / qx, 1.0f);
-        }
-        __syncthreads();
-        const bool take = take_s;
-        __syncthreads();
-        if (take) {
+        const float px = pd[dtok], qx = qd[dtok];
+        if (qx > 0.0f && rng_uniform(st) < (double)fminf(px / qx, 1.0f)) {
             if (threadIdx.x == 0) out[ne] = dtok;
             ne++;
             accepted++;
             continue;
         }
-        // the part of p that q under-covers, in token order
-        float rs = 0.0f;
-        int rc = 0;
-        ordered_scan<256>(vocab, stage, [&](int i) { return pd[i] > qd[i] ? pd[i] - qd[i] : 0.0f; },
-                          [&](int i, float v) {
-                              if (pd[i] > qd[i]) {
-                                  rs += v;
-                                  rc++;
-                              }
-                              return false;
-                          });
-        if (threadIdx.x == 0) stage[256] = (float)rc;
-        __syncthreads();
-        const bool any = stage[256] > 0.0f;
-        __syncthreads();
-        uint32_t t = 0;
-        float u = 0.0f;
-        if (any) {
-            if (threadIdx.x == 0) u = (float)rng_uniform(st) * rs;
-            ordered_scan<256>(vocab, stage, [&](int i) { return pd[i] > qd[i] ? pd[i] - qd[i] : 0.0f; },
-                              [&](int i, float v) {
-                                  if (pd[i] > qd[i]) {
-                                      t = (uint32_t)i;  // the last residual token if u never falls below
-                                      if (u < v) return true;
-                                      u -= v;
-                                  }
-                                  return false;
-                              });
-        } else {
-            // dense_pairs(p): its positive entries in token order
-            float ps = 0.0f;
-            ordered_scan<256>(vocab, stage, [&](int i) { return pd[i]; }, [&](int, float v) {
-                if (v > 0.0f) ps += v;
-                return false;
-            });
-            if (threadIdx.x == 0) u = (float)rng_uniform(st) * ps;
-            ordered_scan<256>(vocab, stage, [&](int i) { return pd[i]; }, [&](int i, float v) {
-                if (v > 0.0f) {
-                    t = (uint32_t)i;
-                    if (u < v) return true;
-                    u -= v;
-                }
-                return false;
-            });
-        }
+        // the part of p that q under-covers, in token order, where there is one
+        int any = 0;
+        for (int i = threadIdx.x; i < vocab; i += blockDim.x) any |= pd[i] > qd[i];
+        any = __syncthreads_or(any);
+        uint32_t t;
+        if (any)
+            t = draw([&](int i) { return pd[i] > qd[i] ? pd[i] - qd[i] : 0.0f; });
+        else
+            t = draw([&](int i) { return pd[i] > 0.0f ? pd[i] : 0.0f; });  // p's positive entries
         if (threadIdx.x == 0) out[ne] = t;
         ne++;
         break;
@@ -650,7 +629,7 @@ __global__ __launch_bounds__(256) void k_accept_wide(int n_seqs, int k, int voca
     if (accepted == k) {
         const int row = sq * K1 + k;
         const size_t pb = (size_t)row * p.cap;
-        const uint32_t t = draw_wide(p.tok + pb, p.pr + pb, p.n[row], st, stage);
+        const uint32_t t = draw_wide(p.tok + pb, p.pr + pb, p.n[row], st, sh);
         if (threadIdx.x == 0) out[ne] = t;
         ne++;
     }
@@ -666,8 +645,14 @@ void launch_dist(hipStream_t st, const float* logits, int rows, int vocab, int r
     if (rows <= 0) return;
     hipLaunchKernelGGL(k_dist, dim3(rows), dim3(kSampleCap), 0, st, logits, vocab, rows_per_seq, prm, out.tok, out.pr,
                        out.tok_id, out.pr_id, out.n, out.cap);
-    if (out.dense) hipLaunchKernelGGL(k_dist_wide, dim3(rows), dim3(kWideThreads), 0, st, logits, vocab, rows_per_seq,
-                                      prm, out);
+    if (!out.dense) return;
+    const dim3 grid((vocab + kWideTile - 1) / kWideTile, rows), block(kWideTile);
+    hipLaunchKernelGGL(k_wide_keys, grid, block, 0, st, logits, vocab, rows_per_seq, prm, out);
+    for (int pass = 0; pass < 4; pass++)
+        hipLaunchKernelGGL(k_wide_sort, grid, block, 0, st, vocab, pass, rows_per_seq, prm, out);
+    hipLaunchKernelGGL(k_wide_exp, grid, block, 0, st, vocab, rows_per_seq, prm, out);
+    hipLaunchKernelGGL(k_wide_sums, dim3(rows), dim3(1024), 0, st, vocab, rows_per_seq, prm, out);
+    hipLaunchKernelGGL(k_wide_pairs, grid, block, 0, st, rows_per_seq, prm, out);
 }
 
 void launch_draw(hipStream_t st, int rows, const SampleParams* prm, const SampleRows& d, uint64_t* rng, uint32_t* out,
@@ -675,7 +660,8 @@ void launch_draw(hipStream_t st, int rows, const SampleParams* prm, const Sample
     if (rows <= 0) return;
     hipLaunchKernelGGL(k_draw, dim3((rows + 63) / 64), dim3(64), 0, st, rows, prm, d.tok, d.pr, d.n, rng, out,
                        out_stride, out_off, d.cap);
-    if (d.dense) hipLaunchKernelGGL(k_draw_wide, dim3(rows), dim3(256), 0, st, rows, prm, d, rng, out, out_stride, out_off);
+    if (d.dense) hipLaunchKernelGGL(k_draw_wide, dim3(rows), dim3(1024), 0, st, rows, prm, d, rng, out, out_stride,
+                                    out_off);
 }
 
 void launch_accept_sampled(hipStream_t st, int n_seqs, int k, const SampleParams* prm, const uint32_t* vtok,
@@ -685,7 +671,7 @@ void launch_accept_sampled(hipStream_t st, int n_seqs, int k, const SampleParams
                        p.pr, p.tok_id, p.pr_id, p.n, q.tok_id, q.pr_id, q.n, rng, out_tokens, out_count,
                        out_accepted, p.cap);
     if (p.dense)
-        hipLaunchKernelGGL(k_accept_wide, dim3(n_seqs), dim3(256), 0, st, n_seqs, k, p.vocab, prm, vtok, am, p, q, rng,
+        hipLaunchKernelGGL(k_accept_wide, dim3(n_seqs), dim3(1024), 0, st, n_seqs, k, p.vocab, prm, vtok, am, p, q, rng,
                            out_tokens, out_count, out_accepted);
 }
 
