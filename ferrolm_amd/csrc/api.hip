@@ -1962,7 +1962,7 @@ int fg_quantize(fg_ctx* ctx, int32_t kind, int32_t rows, int32_t cols, const flo
         return rc;
     HIPCHK(hipMemcpyAsync(dw.p, w, n * 4, hipMemcpyHostToDevice, st));
     if (importance) HIPCHK(hipMemcpyAsync(di.p, importance, (size_t)cols * 4, hipMemcpyHostToDevice, st));
-    launch_quantize(st, kind, rows, cols, dw.f(), importance ? di.f() : nullptr, dq.u8(), ds.f());
+    launch_quantize(st, kind, rows, cols, dw.f(), nullptr, importance ? di.f() : nullptr, dq.u8(), nullptr, ds.f());
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(q, dq.p, qb, hipMemcpyDeviceToHost, st));
     HIPCHK(hipMemcpyAsync(s, ds.p, sn * 4, hipMemcpyDeviceToHost, st));
@@ -1980,64 +1980,59 @@ int fg_awq_search(fg_ctx* ctx, int32_t kind, int32_t rows, int32_t k, const floa
     hipStream_t st = ctx->stream;
     const size_t rk = (size_t)rows * k, mk = (size_t)m * k, ny = (size_t)m * rows;
     const size_t qb = kind == FG_INT8 ? rk : rk / 2, sn = rk / 32;
-    // channel statistics on the host (f64 sums in row order)
-    std::vector<float> am(k), sq(k), sc(k), imp(k), best_s(k);
-    fh_awq_stats(cal, m, k, am.data(), sq.data());
+    // channel statistics on the host (f64 sums in row order), and every alpha's scales and
+    // importances imp = sq / s^2 + 1e-8 (apply, src/awq.rs:152-165)
     constexpr int kSteps = 11;  // alpha = 0, 0.1, ..., 1
-    DevBuf dw, dws, dx, dxs, dyref, dy, dsc, dimp, dq, ds, derr;
-    if ((rc = dev_alloc(dw, rk * 4)) || (rc = dev_alloc(dws, rk * 4)) || (rc = dev_alloc(dx, mk * 4)) ||
+    std::vector<float> am(k), sq(k), host((size_t)kSteps * 2 * k);
+    fh_awq_stats(cal, m, k, am.data(), sq.data());
+    auto scales_of = [&](int step) { return host.data() + (size_t)step * 2 * k; };
+    for (int step = 0; step < kSteps; step++) {
+        float *sv = scales_of(step), *imp = sv + k;
+        fh_awq_scales(am.data(), k, (float)step / 10.0f, sv);
+        for (int32_t c = 0; c < k; c++) imp[c] = sq[c] / (sv[c] * sv[c]) + 1e-8f;
+    }
+    DevBuf dw, dwt, dx, dxs, dyref, dy, dsc, dq, ds, derr, dwork;
+    if ((rc = dev_alloc(dw, rk * 4)) || (rc = dev_alloc(dwt, rk * 2)) || (rc = dev_alloc(dx, mk * 4)) ||
         (rc = dev_alloc(dxs, mk * 4)) || (rc = dev_alloc(dyref, ny * 4)) || (rc = dev_alloc(dy, kSteps * ny * 4)) ||
-        (rc = dev_alloc(dsc, (size_t)k * 4)) || (rc = dev_alloc(dimp, (size_t)k * 4)) || (rc = dev_alloc(dq, qb)) ||
-        (rc = dev_alloc(ds, sn * 4)) || (rc = dev_alloc(derr, kSteps * 8)))
+        (rc = dev_alloc(dsc, host.size() * 4)) || (rc = dev_alloc(dq, qb)) || (rc = dev_alloc(ds, sn * 4)) ||
+        (rc = dev_alloc(derr, kSteps * 8)) || (rc = dev_alloc(dwork, sq_err_work(kSteps, (int64_t)ny))))
         return rc;
     HIPCHK(hipMemcpyAsync(dw.p, w, rk * 4, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(dx.p, cal, mk * 4, hipMemcpyHostToDevice, st));
+    HIPCHK(hipMemcpyAsync(dsc.p, host.data(), host.size() * 4, hipMemcpyHostToDevice, st));
     // the reference output, with the unquantized weights as bf16 (Matrix::from_f32)
-    launch_mm_exact(st, BF16, dx.f(), m, k, dw.f(), nullptr, nullptr, rows, dyref.f());
-    HIPCHK(hipGetLastError());
-    // imp = sq / s^2 + 1e-8 and the scaled operands, then the quantizer (apply, src/awq.rs:152-165)
-    auto apply = [&](const float* sv) -> int {
-        for (int32_t c = 0; c < k; c++) imp[c] = sq[c] / (sv[c] * sv[c]) + 1e-8f;
-        HIPCHK(hipMemcpyAsync(dsc.p, sv, (size_t)k * 4, hipMemcpyHostToDevice, st));
-        HIPCHK(hipMemcpyAsync(dimp.p, imp.data(), (size_t)k * 4, hipMemcpyHostToDevice, st));
-        launch_scale_cols(st, dw.f(), (int64_t)rk, k, dsc.f(), 0, dws.f());
-        launch_quantize(st, kind, rows, k, dws.f(), dimp.f(), dq.u8(), ds.f());
-        HIPCHK(hipGetLastError());
-        return 0;
-    };
+    uint32_t* wt = (uint32_t*)dwt.p;
+    launch_pack_bf16(st, dw.f(), rows, k, wt);
+    launch_mm_exact(st, BF16, dx.f(), m, k, wt, nullptr, rows, dyref.f());
     // every alpha's product first, then their error sums side by side
-    std::vector<std::vector<float>> scs(kSteps);
     for (int step = 0; step < kSteps; step++) {
-        scs[step].resize(k);
-        fh_awq_scales(am.data(), k, (float)step / 10.0f, scs[step].data());
-        if ((rc = apply(scs[step].data()))) return rc;
-        launch_scale_cols(st, dx.f(), (int64_t)mk, k, dsc.f(), 1, dxs.f());
-        launch_mm_exact(st, kind, dxs.f(), m, k, nullptr, dq.u8(), ds.f(), rows, dy.f() + (size_t)step * ny);
-        HIPCHK(hipGetLastError());
-        // the scales and importance buffers are rewritten by the next step's copies
-        HIPCHK(hipStreamSynchronize(st));
+        const float *sv = dsc.f() + (size_t)step * 2 * k, *imp = sv + k;
+        launch_quantize(st, kind, rows, k, dw.f(), sv, imp, nullptr, wt, ds.f());
+        launch_scale_cols(st, dx.f(), (int64_t)mk, k, sv, dxs.f());
+        launch_mm_exact(st, kind, dxs.f(), m, k, wt, ds.f(), rows, dy.f() + (size_t)step * ny);
     }
-    launch_sq_err(st, dy.f(), (int64_t)ny, kSteps, dyref.f(), (int64_t)ny, (double*)derr.p);
+    launch_sq_err(st, dy.f(), (int64_t)ny, kSteps, dyref.f(), (int64_t)ny, dwork.p, (double*)derr.p);
     HIPCHK(hipGetLastError());
     double errs[kSteps];
     HIPCHK(hipMemcpyAsync(errs, derr.p, sizeof(errs), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     double best = INFINITY, plain = errs[0];
-    float best_alpha = 0.0f;
+    int best_step = 0;
     bool have = false;
     for (int step = 0; step < kSteps; step++)
         if (!have || errs[step] < best) {  // the first minimum, as the reference's search
             have = true;
             best = errs[step];
-            best_alpha = (float)step / 10.0f;
-            best_s = scs[step];
+            best_step = step;
         }
-    if ((rc = apply(best_s.data()))) return rc;
+    const float* bs = dsc.f() + (size_t)best_step * 2 * k;
+    launch_quantize(st, kind, rows, k, dw.f(), bs, bs + k, dq.u8(), nullptr, ds.f());
+    HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(q, dq.p, qb, hipMemcpyDeviceToHost, st));
     HIPCHK(hipMemcpyAsync(s, ds.p, sn * 4, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
-    std::memcpy(scales, best_s.data(), (size_t)k * 4);
-    choice->alpha = best_alpha;
+    std::memcpy(scales, scales_of(best_step), (size_t)k * 4);
+    choice->alpha = (float)best_step / 10.0f;
     choice->_pad = 0;
     choice->error_plain = plain;
     choice->error_awq = best;

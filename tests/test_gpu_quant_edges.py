@@ -1,0 +1,46 @@
+"""The quantizer and the AWQ search where their shortcuts end: weights on and
+next to rounding boundaries of their scale, empty groups, magnitudes at the ends
+of the f32 range, and error sums of a chunk less, exactly and more than a chunk
+(8192 terms). Codes, scales and errors equal the oracle's bit for bit."""
+import numpy as np
+import pytest
+
+import oracle
+from ferrolm_amd import gpu
+from ferrolm_amd.weights import INT4, INT8
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind", [INT8, INT4], ids=["int8", "int4"])
+@pytest.mark.parametrize("case", ["halves", "near halves", "zeros", "tiny", "denormal", "huge", "one value"])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_quantizer_boundaries(ctx, kind, case, weighted):
+    rng = np.random.default_rng(7)
+    hi = 127 if kind == INT8 else 7
+    w = rng.integers(-2 * hi, 2 * hi + 1, (64, 160)).astype(np.float32) / 2  # halves of a code at scale 1
+    w[:, ::32] = hi
+    if case == "near halves":
+        w = np.nextafter(w, np.where(rng.random(w.shape) < 0.5, -np.inf, np.inf).astype(np.float32))
+    elif case == "zeros":
+        w[::3] = 0
+        w[:, 32:64] = 0
+    elif case in ("tiny", "denormal", "huge"):
+        w = w * np.float32({"tiny": 1e-33, "denormal": 1e-41, "huge": 1e36}[case])
+    elif case == "one value":
+        w = np.full_like(w, -0.7)
+    imp = rng.random(160).astype(np.float32) if weighted else None
+    got, want = gpu.quantize(ctx, kind, w, imp), oracle.quantize(kind, w, imp)
+    assert np.array_equal(got.s, want.s)
+    assert np.array_equal(got.q, want.q)
+
+
+@pytest.mark.parametrize("rows,m", [(32, 1), (32, 255), (32, 256), (32, 257), (288, 91)])
+def test_search_errors_across_chunks(ctx, rows, m):
+    rng = np.random.default_rng(rows + m)
+    w = (0.02 * rng.standard_normal((rows, 160))).astype(np.float32)
+    cal = rng.standard_normal((m, 160)).astype(np.float32) * np.exp(2 * rng.standard_normal((m, 1))).astype(np.float32)
+    got, want = gpu.awq_search(ctx, INT4, w, cal), oracle.awq_search(INT4, w, cal)
+    assert got[1:4] == tuple(want[1:4])
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[4].q, want[4].q)
+    assert np.array_equal(got[4].s, want[4].s)
