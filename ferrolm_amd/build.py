@@ -24,7 +24,11 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 OBJ = PKG / "_build"
 LIB = PKG / "libferro_gpu.so"
-SOURCES = ["kernels.hip", "sampling.hip", "quant.hip", "api.hip"]
+SOURCES = ["kernels.hip", "gemm.hip", "gemm_bf16.hip", "gemm_int8.hip", "gemm_int4.hip", "sampling.hip", "quant.hip", "api.hip"]
+# MFMA results in VGPRs: where a workgroup fills a CU's LDS a wave may take 512 registers, and the
+# compiler would put every product into the accumulation registers and copy it out again for the VALU
+MFMA_IN_VGPRS = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
+EXTRA_FLAGS = {f"gemm_{k}.hip": MFMA_IN_VGPRS for k in ("bf16", "int8", "int4")}
 HOST_SOURCES = ["host.cpp"]  # plain C++ (g++), no contraction: exact load-time arithmetic
 ARCH = os.environ.get("FERRO_OFFLOAD_ARCH", "gfx950")
 
@@ -51,7 +55,7 @@ def build(verbose: bool = False, stamps: bool = False) -> Path:
 
     def compile_one(src: str) -> Path:
         out = obj / (Path(src).stem + ".o")
-        cmd = [cc, *flags(), *extra, "-c", str(CSRC / src), "-o", str(out)]
+        cmd = [cc, *flags(), *EXTRA_FLAGS.get(src, []), *extra, "-c", str(CSRC / src), "-o", str(out)]
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"hipcc failed on {src}:\n{r.stderr}")

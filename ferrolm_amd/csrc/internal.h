@@ -180,6 +180,9 @@ struct GemvArgs {
 // so their interval is the kernel's own execution time.
 void launch_gemv(hipStream_t st, int epi, const DMat& w, const GemvArgs& a, hipEvent_t start = nullptr,
                  hipEvent_t stop = nullptr);
+// The tiled GEMM (gemm.hip) for MM inputs: 1, or 0 when the product is not its size and nothing
+// was launched.
+int launch_mm(hipStream_t st, int epi, const DMat& w, const GemvArgs& a, hipEvent_t e0, hipEvent_t e1);
 // The output projection of a fused bf16 layer split by query head (k_o_heads):
 // a.apart / a.amrec the attention's span partials and merge records, a.anh,
 // a.ankv, a.ahd, a.aqm their geometry; the product is added into a.acc_out and

@@ -1453,6 +1453,8 @@ static void gemm_rtw(hipStream_t st, int epi, const DMat& w, const GemvArgs& a0,
 
 template <int KIND>
 static void gemm_kind(hipStream_t st, int epi, const DMat& w, const GemvArgs& a, hipEvent_t e0, hipEvent_t e1) {
+    // the tiled GEMM (gemm.hip) takes the products whose tiles fill the chip; what is left:
+    if (launch_mm(st, epi, w, a, e0, e1)) return;
     const int rt = (a.p_total + 3) / 4, groups = (rt + 4) / 5, rtw = (rt + groups - 1) / groups;
     // 128-column tiles (CS 2) for steps of 256 rows or more when they still make
     // 512 workgroups (measured on the 1.7B int4 prefill of 1024 tokens: 14.45

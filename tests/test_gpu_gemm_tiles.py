@@ -1,0 +1,104 @@
+"""The tiled GEMM at the edges of its tiles: one product for each tile shape,
+with outputs that are not a multiple of 64 or 128, rows that are not one of 16,
+an input of 5 k-blocks (padded to 8, so some shares of K have one stage and some
+none left) and one of 35 (padded to 36: a last stage that is not full); outputs
+into a buffer aligned to a float only; and a forward whose projections take it
+with every epilogue.
+
+A product's rows are held as two bf16 pieces (2^-17 of each input) and summed in
+f32, so |y - exact| <= 2e-5 * sum|x||w| as in the other products' tests."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle
+from ferrolm_amd import gpu
+from ferrolm_amd.weights import BF16, INT4, INT8, Config, Matrix
+
+from test_zz_no_alloc import Hip
+
+pytestmark = pytest.mark.gpu
+
+# (outputs, inputs, rows): the shape's tile of row tiles x 64-column waves x K shares
+SHAPES = [(10016, 160, 1000),   # 8 x 4 x 1
+          (16448, 160, 400),    # 5 x 4 x 1
+          (9440, 160, 517),     # 8 x 4 x 2
+          (16448, 160, 200),    # 5 x 2 x 2
+          (16448, 160, 83),     # 4 x 2 x 2
+          (11456, 160, 129),    # 5 x 2 x 4
+          (6560, 160, 200),     # 4 x 2 x 4
+          (11456, 160, 67),     # 3 x 2 x 4
+          (1856, 1120, 300),    # 2 x 2 x 4
+          (16448, 1120, 200), (11456, 1120, 129), (6560, 1120, 200)]
+
+
+def _matrix(kind, n, k, rng):
+    w = (0.1 * rng.standard_normal((n, k))).astype(np.float32)
+    if kind == BF16:
+        return Matrix(BF16, n, k, bf16=(w.view(np.uint32) >> 16).astype(np.uint16))
+    return oracle.quantize(kind, w)
+
+
+@pytest.mark.parametrize("kind", [BF16, INT8, INT4], ids=["bf16", "int8", "int4"])
+@pytest.mark.parametrize("n,k,m", SHAPES)
+def test_products_of_every_tile_shape(ctx, kind, n, k, m):
+    rng = np.random.default_rng(n + k + m)
+    w = _matrix(kind, n, k, rng)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[:, ::7] *= 20.0
+    b = rng.standard_normal(n).astype(np.float32)
+    y = gpu.Mat(ctx, w).matmul(x, b)
+    deq = w.to_f32().astype(np.float64)
+    scale = np.abs(x).astype(np.float64) @ np.abs(deq).T
+    assert np.all(np.abs(y - (x.astype(np.float64) @ deq.T + b)) <= 2e-5 * scale + 1e-6)
+
+
+def test_output_aligned_to_a_float(ctx):
+    hip = Hip()
+    rng = np.random.default_rng(1)
+    n, k, m = 6560, 160, 200
+    w = gpu.Mat(ctx, _matrix(INT4, n, k, rng))
+    xh = rng.standard_normal((m, k)).astype(np.float32)
+    x, y = hip.alloc(xh.nbytes), hip.alloc(4 * (m * n + 8))
+    got = []
+    try:
+        hip.put(x, xh)
+        for off in (0, 1):
+            hip.put(y, np.full(m * n + 8, 7.0, np.float32))
+            gpu.check(gpu.lib().fg_matmul_device(ctx.h, w.h, x, m, C.c_void_p(y.value + 4 * off)))
+            ctx.sync()
+            got.append(hip.get(y, m * n + 8))
+    finally:
+        hip.free(x, y)
+    assert np.array_equal(got[0][:m * n], got[1][1:m * n + 1])
+    assert got[1][0] == 7.0 and np.all(got[1][m * n + 1:] == 7.0)
+
+
+@pytest.mark.parametrize("kind", [BF16, INT8, INT4], ids=["bf16", "int8", "int4"])
+def test_forward_on_the_tiles_matches_oracle(ctx, kind):
+    """600 rows of a 1056-wide model (33 k-blocks, padded to 36), two layers: q/k/v with a bias, o, gate/up,
+    down (two k-blocks of padding after its output) and the lm_head, logits, hidden states and cache slots
+    within 1e-4 of the oracle."""
+    from ferrolm_amd.synth import quantize_model, random_model
+    cfg = Config(vocab=6560, hidden=1056, intermediate=4256, layers=2, heads=33, kv_heads=11, head_dim=32,
+                 rms_eps=1e-5, max_position=1024, qkv_bias=True)
+    hm = quantize_model(random_model(cfg, seed=7, std=0.03), kind)
+    n = 600
+    prompt = [int(t) for t in np.random.default_rng(8).integers(0, cfg.vocab, n)]
+    blocks = (n + 15) // 16
+    table = [(i * 7) % blocks for i in range(blocks)]
+    m, kv = gpu.Model(ctx, hm), gpu.KvCache(ctx, cfg, blocks)
+    out = gpu.forward(ctx, m, kv, [(prompt, 0, table, gpu.LOGITS_ALL)], hidden=True)
+    om = oracle.Model(hm)
+    okv = om.kv(blocks)
+    ol, oh = om.forward(okv, [(prompt, 0, table, 2)], hidden=True)
+    assert np.abs(out.logits - ol).max() < 1e-4 * np.abs(ol).max()
+    rel = np.linalg.norm(out.hidden - oh, axis=-1) / np.linalg.norm(oh, axis=-1)
+    assert rel.max() < 1e-4, rel.max()
+    top2 = np.sort(ol, axis=1)[:, -2:]
+    clear = top2[:, 1] - top2[:, 0] > 2e-4 * np.abs(ol).max()
+    assert clear.mean() > 0.9 and np.array_equal(out.argmax[clear], ol.argmax(axis=1)[clear])
+    for li in range(cfg.layers):
+        for g, o in zip(kv.layer(li), okv.layer(li)):
+            assert np.abs(g - o).max() <= 1e-4 * np.abs(o).max()
