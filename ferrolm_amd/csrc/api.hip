@@ -7,12 +7,12 @@
 #include "internal.h"
 
 #include <algorithm>
-#include <mutex>
 #include <atomic>
 #include <cstdlib>
 #include <functional>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -74,6 +74,36 @@ struct Carver {
 // ---------------------------------------------------------------------------
 // Handles
 // ---------------------------------------------------------------------------
+// Staging of large host copies (copy_host, quantize_staged): kSlots slots, each a pinned and a
+// device region for kSlotIn bytes of input and kSlotOut of output; a worker thread t owns slots
+// t * kSlotsEach ... and streams[t]. Made by the first call that wants it, freed with
+// the context.
+struct Stage {
+    static constexpr int kThreads = 4, kSlotsEach = 2, kSlots = kThreads * kSlotsEach;
+    static constexpr size_t kSlotIn = (size_t)4 << 20, kSlotOut = (size_t)1280 << 10;
+    static constexpr size_t kCopyMin = (size_t)4 << 20, kPanelsMin = (size_t)16 << 20;
+    char *pin = nullptr, *dev = nullptr;
+    hipStream_t streams[kThreads] = {};
+    hipEvent_t ev[kSlots] = {};
+    std::mutex mu;  // one call at a time
+    char* pin_in(int i) const { return pin + i * kSlotIn; }
+    char* pin_out(int i) const { return pin + kSlots * kSlotIn + i * kSlotOut; }
+    char* dev_in(int i) const { return dev + i * kSlotIn; }
+    char* dev_out(int i) const { return dev + kSlots * kSlotIn + i * kSlotOut; }
+};
+
+static void stage_free(Stage& g) {
+    if (g.pin) (void)hipHostFree(g.pin);
+    if (g.dev) (void)hipFree(g.dev);
+    for (auto& x : g.streams)
+        if (x) (void)hipStreamDestroy(x);
+    for (auto& e : g.ev)
+        if (e) (void)hipEventDestroy(e);
+    g.pin = g.dev = nullptr;
+    for (auto& x : g.streams) x = nullptr;
+    for (auto& e : g.ev) e = nullptr;
+}
+
 struct fg_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -88,6 +118,7 @@ struct fg_ctx {
     size_t dmeta_cap = 0;
     void* hmeta = nullptr;
     size_t hmeta_cap = 0;
+    Stage stage;  // slots for large host copies of load-time calls
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
     float last_us[3] = {0, 0, 0};
     bool merge_in_o = true;  // small bf16 output projections merge the attention spans themselves
@@ -1059,6 +1090,139 @@ static int run_forward(fg_ctx* ctx, const fg_model* m, fg_kv* kv, const Plan& P,
 }
 
 // ---------------------------------------------------------------------------
+// Large host copies of the load-time calls
+// ---------------------------------------------------------------------------
+
+namespace {
+// A device allocation freed when it leaves scope (hipFree waits for the
+// device, so queued work that uses it has finished).
+struct DevBuf {
+    void* p = nullptr;
+    DevBuf() = default;
+    DevBuf(const DevBuf&) = delete;
+    ~DevBuf() {
+        if (p) (void)hipFree(p);
+    }
+};
+}  // namespace
+
+static int dev_alloc(DevBuf& b, size_t bytes) {
+    if (hipMalloc(&b.p, std::max<size_t>(bytes, 256)) != hipSuccess) {
+        b.p = nullptr;
+        (void)hipGetLastError();
+        return fail(FG_E_NOMEM, "device allocation failed");
+    }
+    return 0;
+}
+
+// False when the slots can't be had (the caller then copies without them).
+static bool stage_ready(Stage& g) {
+    if (g.pin) return true;
+    const size_t bytes = Stage::kSlots * (Stage::kSlotIn + Stage::kSlotOut);
+    bool ok = hipHostMalloc((void**)&g.pin, bytes, hipHostMallocDefault) == hipSuccess;
+    if (!ok) g.pin = nullptr;
+    if (ok && hipMalloc((void**)&g.dev, bytes) != hipSuccess) {
+        ok = false;
+        g.dev = nullptr;
+    }
+    for (auto& x : g.streams)
+        if (ok && hipStreamCreateWithFlags(&x, hipStreamNonBlocking) != hipSuccess) {
+            ok = false;
+            x = nullptr;
+        }
+    for (auto& e : g.ev)
+        if (ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+            ok = false;
+            e = nullptr;
+        }
+    if (!ok) {
+        (void)hipGetLastError();
+        stage_free(g);
+    }
+    return ok;
+}
+
+// Runs issue(chunk, slot, stream) -> hipError_t for every chunk, on up to kThreads threads with
+// slots of their own, and finish(chunk, slot) once what issue queued on the stream is done.
+// Returns with nothing left in flight.
+template <class I, class F>
+static int staged(fg_ctx* c, size_t chunks, const I& issue, const F& finish) {
+    Stage& g = c->stage;
+    std::atomic<size_t> next{0};
+    std::atomic<bool> bad{false};
+    auto work = [&](int t) {
+        hipStream_t st = g.streams[t];
+        if (hipSetDevice(c->device) != hipSuccess) bad = true;
+        size_t held[Stage::kSlotsEach] = {};  // chunk + 1
+        auto drain = [&](int k) {
+            if (!held[k]) return;
+            const int slot = t * Stage::kSlotsEach + k;
+            if (hipEventSynchronize(g.ev[slot]) != hipSuccess) bad = true;
+            if (!bad) finish(held[k] - 1, slot);
+            held[k] = 0;
+        };
+        int k = 0;
+        for (; !bad; k = (k + 1) % Stage::kSlotsEach) {
+            drain(k);
+            const size_t ch = next++;
+            if (ch >= chunks) break;
+            const int slot = t * Stage::kSlotsEach + k;
+            if (issue(ch, slot, st) != hipSuccess || hipEventRecord(g.ev[slot], st) != hipSuccess) bad = true;
+            held[k] = ch + 1;
+        }
+        for (int j = 0; j < Stage::kSlotsEach; j++) drain((k + j) % Stage::kSlotsEach);
+    };
+    std::thread th[Stage::kThreads];
+    int nt = (int)std::min<size_t>(std::min(Stage::kThreads, std::max(1, (int)std::thread::hardware_concurrency())), chunks);
+    for (int t = 1; t < nt; t++) {
+        try {
+            th[t] = std::thread(work, t);
+        } catch (...) {  // no more threads to be had: the others take its chunks
+            break;
+        }
+    }
+    work(0);
+    for (auto& x : th)
+        if (x.joinable()) x.join();
+    if (bad) {
+        for (auto& x : g.streams) (void)hipStreamSynchronize(x);
+        (void)hipGetLastError();
+        return fail(FG_E_DEVICE, "staged copy failed");
+    }
+    return 0;
+}
+
+// A copy between pageable host memory and the device that is complete on return. The runtime's
+// own copy of pageable memory ran at 28 GB/s and one thread's memcpy into pinned memory at 32,
+// pinned memory to the device at 56, so slots filled by several threads keep the link busy. A
+// thread gets about eight chunks: fewer leave the link idle at both ends (50 MB took 2.05 ms in
+// chunks of 4 MB; 0.5 less in chunks of 1.5), and below 512 KB a chunk's calls cost more than its
+// bytes.
+static int copy_host(fg_ctx* c, void* dst, const void* src, size_t bytes, bool to_device) {
+    const hipMemcpyKind kind = to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
+    if (bytes < Stage::kCopyMin || !stage_ready(c->stage)) {
+        HIPCHK(hipMemcpyAsync(dst, src, bytes, kind, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        return 0;
+    }
+    HIPCHK(hipStreamSynchronize(c->stream));  // the slots' streams wait for nothing else
+    const Stage& g = c->stage;
+    const size_t part = std::min(Stage::kSlotIn, std::max((size_t)512 << 10, (bytes / (8 * Stage::kThreads) + 4095) & ~(size_t)4095));
+    auto len = [&](size_t ch) { return std::min(part, bytes - ch * part); };
+    return staged(
+        c, (bytes + part - 1) / part,
+        [&](size_t ch, int slot, hipStream_t st) {
+            const size_t o = ch * part;
+            if (!to_device) return hipMemcpyAsync(g.pin_in(slot), (const char*)src + o, len(ch), kind, st);
+            std::memcpy(g.pin_in(slot), (const char*)src + o, len(ch));
+            return hipMemcpyAsync((char*)dst + o, g.pin_in(slot), len(ch), kind, st);
+        },
+        [&](size_t ch, int slot) {
+            if (!to_device) std::memcpy((char*)dst + ch * part, g.pin_in(slot), len(ch));
+        });
+}
+
+// ---------------------------------------------------------------------------
 // C ABI
 // ---------------------------------------------------------------------------
 extern "C" {
@@ -1129,6 +1293,7 @@ void fg_ctx_destroy(fg_ctx* c) {
     if (c->sbuf) (void)hipFree(c->sbuf);
     if (c->dmeta) (void)hipFree(c->dmeta);
     if (c->hmeta) (void)hipHostFree(c->hmeta);
+    stage_free(c->stage);
     if (c->gcnt) (void)hipFree(c->gcnt);
     for (auto& e : c->ev)
         if (e) (void)hipEventDestroy(e);
@@ -1917,30 +2082,6 @@ int fg_matmul_device_noalloc(fg_ctx* ctx, const fg_mat* w, const float* x_dev, i
 
 // ---- load-time quantization on the device --------------------------------
 
-namespace {
-// A device allocation freed when it leaves scope (hipFree waits for the
-// device, so queued work that uses it has finished).
-struct DevBuf {
-    void* p = nullptr;
-    DevBuf() = default;
-    DevBuf(const DevBuf&) = delete;
-    ~DevBuf() {
-        if (p) (void)hipFree(p);
-    }
-    float* f() const { return (float*)p; }
-    uint8_t* u8() const { return (uint8_t*)p; }
-};
-}  // namespace
-
-static int dev_alloc(DevBuf& b, size_t bytes) {
-    if (hipMalloc(&b.p, std::max<size_t>(bytes, 256)) != hipSuccess) {
-        b.p = nullptr;
-        (void)hipGetLastError();
-        return fail(FG_E_NOMEM, "device allocation failed");
-    }
-    return 0;
-}
-
 static int quant_shape(int32_t kind, int32_t rows, int32_t cols) {
     if (kind != FG_INT8 && kind != FG_INT4) return fail(FG_E_ARG, "format must be FG_INT8 or FG_INT4");
     if (rows <= 0 || cols <= 0) return fail(FG_E_ARG, "empty matrix");
@@ -1955,19 +2096,59 @@ int fg_quantize(fg_ctx* ctx, int32_t kind, int32_t rows, int32_t cols, const flo
     if ((rc = quant_shape(kind, rows, cols))) return rc;
     HIPCHK(hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
+    std::lock_guard<std::mutex> one(ctx->stage.mu);
     const size_t n = (size_t)rows * cols, qb = kind == FG_INT8 ? n : n / 2, sn = n / 32;
-    DevBuf dw, di, dq, ds;
-    if ((rc = dev_alloc(dw, n * 4)) || (rc = dev_alloc(di, (size_t)cols * 4)) || (rc = dev_alloc(dq, qb)) ||
-        (rc = dev_alloc(ds, sn * 4)))
-        return rc;
-    HIPCHK(hipMemcpyAsync(dw.p, w, n * 4, hipMemcpyHostToDevice, st));
-    if (importance) HIPCHK(hipMemcpyAsync(di.p, importance, (size_t)cols * 4, hipMemcpyHostToDevice, st));
-    launch_quantize(st, kind, rows, cols, dw.f(), nullptr, importance ? di.f() : nullptr, dq.u8(), nullptr, ds.f());
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(q, dq.p, qb, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(s, ds.p, sn * 4, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    return 0;
+    const size_t panel = (size_t)32 * cols, ib = importance ? (size_t)cols * 4 : 0;  // a panel of 32 rows is on its own
+    auto apart = [&](const void* o, size_t bytes) {  // results come back while weights are still being read
+        return (const char*)o + bytes <= (const char*)w || (const char*)w + n * 4 <= (const char*)o;
+    };
+    const bool split = n * 4 >= Stage::kPanelsMin && panel * 4 <= Stage::kSlotIn && apart(q, qb) && apart(s, sn * 4) &&
+                       stage_ready(ctx->stage);
+    float *dw, *di, *ds;
+    uint8_t* dq;
+    auto layout = [&](void* base) {
+        Carver cv(base);
+        di = cv.take<float>(ib / 4);
+        dw = cv.take<float>(split ? 0 : n);
+        dq = cv.take<uint8_t>(split ? 0 : qb);
+        ds = cv.take<float>(split ? 0 : sn);
+        return cv.off;
+    };
+    DevBuf buf;
+    if ((rc = dev_alloc(buf, layout(nullptr)))) return rc;
+    layout(buf.p);
+    if (importance && (rc = copy_host(ctx, di, importance, ib, true))) return rc;
+    if (!split) {
+        if ((rc = copy_host(ctx, dw, w, n * 4, true))) return rc;
+        launch_quantize(st, kind, rows, cols, dw, nullptr, importance ? di : nullptr, dq, nullptr, ds);
+        HIPCHK(hipGetLastError());
+        if ((rc = copy_host(ctx, q, dq, qb, false))) return rc;
+        return copy_host(ctx, s, ds, sn * 4, false);
+    }
+    // Panels go up, are quantized and come back side by side: bound by the link's 56 GB/s up
+    // (16384 x 2048 to int4: 6.8 -> 3.3 ms for the call, 2.4 of them the copy up).
+    const Stage& g = ctx->stage;
+    const int each = (int)(Stage::kSlotIn / (panel * 4)), panels = rows / 32;
+    const size_t pq = qb / panels, ps = cols * 4;  // a panel's codes and scales
+    auto count = [&](size_t ch) { return (size_t)std::min(each, panels - (int)ch * each); };
+    return staged(
+        ctx, (panels + each - 1) / each,
+        [&](size_t ch, int slot, hipStream_t ss) {
+            const size_t np = count(ch), p0 = ch * each;
+            std::memcpy(g.pin_in(slot), w + p0 * panel, np * panel * 4);
+            hipError_t e = hipMemcpyAsync(g.dev_in(slot), g.pin_in(slot), np * panel * 4, hipMemcpyHostToDevice, ss);
+            if (e != hipSuccess) return e;
+            char* out = g.dev_out(slot);
+            launch_quantize(ss, kind, (int)np * 32, cols, (const float*)g.dev_in(slot), nullptr, importance ? di : nullptr,
+                            (uint8_t*)out, nullptr, (float*)(out + np * pq));
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+            return hipMemcpyAsync(g.pin_out(slot), out, np * (pq + ps), hipMemcpyDeviceToHost, ss);
+        },
+        [&](size_t ch, int slot) {
+            const size_t np = count(ch), p0 = ch * each;
+            std::memcpy(q + p0 * pq, g.pin_out(slot), np * pq);
+            std::memcpy((char*)s + p0 * ps, g.pin_out(slot) + np * pq, np * ps);
+        });
 }
 
 int fg_awq_search(fg_ctx* ctx, int32_t kind, int32_t rows, int32_t k, const float* w, int32_t m, const float* cal,
@@ -1984,37 +2165,76 @@ int fg_awq_search(fg_ctx* ctx, int32_t kind, int32_t rows, int32_t k, const floa
     // importances imp = sq / s^2 + 1e-8 (apply, src/awq.rs:152-165)
     constexpr int kSteps = 11;  // alpha = 0, 0.1, ..., 1
     std::vector<float> am(k), sq(k), host((size_t)kSteps * 2 * k);
-    fh_awq_stats(cal, m, k, am.data(), sq.data());
     auto scales_of = [&](int step) { return host.data() + (size_t)step * 2 * k; };
-    for (int step = 0; step < kSteps; step++) {
-        float *sv = scales_of(step), *imp = sv + k;
-        fh_awq_scales(am.data(), k, (float)step / 10.0f, sv);
-        for (int32_t c = 0; c < k; c++) imp[c] = sq[c] / (sv[c] * sv[c]) + 1e-8f;
+    auto statistics = [&] {
+        fh_awq_stats(cal, m, k, am.data(), sq.data());
+        for (int step = 0; step < kSteps; step++) {
+            float *sv = scales_of(step), *imp = sv + k;
+            fh_awq_scales(am.data(), k, (float)step / 10.0f, sv);
+            for (int32_t c = 0; c < k; c++) imp[c] = sq[c] / (sv[c] * sv[c]) + 1e-8f;
+        }
+    };
+    float *dw, *dx, *dxs, *dyref, *dy, *dsc, *ds;
+    uint32_t* wt;
+    uint8_t *dq, *dwork;
+    double* derr;
+    auto layout = [&](void* base) {
+        Carver cv(base);
+        dw = cv.take<float>(rk);
+        wt = cv.take<uint32_t>(rk / 2);
+        dx = cv.take<float>(mk);
+        dxs = cv.take<float>(mk);
+        dyref = cv.take<float>(ny);
+        dy = cv.take<float>(kSteps * ny);
+        dsc = cv.take<float>(host.size());
+        dq = cv.take<uint8_t>(qb);
+        ds = cv.take<float>(sn);
+        derr = cv.take<double>(kSteps);
+        dwork = cv.take<uint8_t>(sq_err_work(kSteps, (int64_t)ny));
+        return cv.off;
+    };
+    std::lock_guard<std::mutex> one(ctx->stage.mu);
+    DevBuf buf;
+    if ((rc = dev_alloc(buf, layout(nullptr)))) return rc;
+    layout(buf.p);
+    {
+        // (256 x 2048: 0.37 ms beside the copies of the rows and the weights)
+        std::atomic<bool> done{false};
+        struct Join {
+            std::thread t;
+            ~Join() {
+                if (t.joinable()) t.join();
+            }
+        } beside;
+        try {
+            beside.t = std::thread([&] {
+                try {
+                    statistics();
+                    done = true;
+                } catch (...) {
+                }
+            });
+        } catch (...) {
+        }
+        if ((rc = copy_host(ctx, dw, w, rk * 4, true)) || (rc = copy_host(ctx, dx, cal, mk * 4, true))) return rc;
+        if (beside.t.joinable()) beside.t.join();
+        if (!done) statistics();
     }
-    DevBuf dw, dwt, dx, dxs, dyref, dy, dsc, dq, ds, derr, dwork;
-    if ((rc = dev_alloc(dw, rk * 4)) || (rc = dev_alloc(dwt, rk * 2)) || (rc = dev_alloc(dx, mk * 4)) ||
-        (rc = dev_alloc(dxs, mk * 4)) || (rc = dev_alloc(dyref, ny * 4)) || (rc = dev_alloc(dy, kSteps * ny * 4)) ||
-        (rc = dev_alloc(dsc, host.size() * 4)) || (rc = dev_alloc(dq, qb)) || (rc = dev_alloc(ds, sn * 4)) ||
-        (rc = dev_alloc(derr, kSteps * 8)) || (rc = dev_alloc(dwork, sq_err_work(kSteps, (int64_t)ny))))
-        return rc;
-    HIPCHK(hipMemcpyAsync(dw.p, w, rk * 4, hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dx.p, cal, mk * 4, hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dsc.p, host.data(), host.size() * 4, hipMemcpyHostToDevice, st));
+    if ((rc = copy_host(ctx, dsc, host.data(), host.size() * 4, true))) return rc;
     // the reference output, with the unquantized weights as bf16 (Matrix::from_f32)
-    uint32_t* wt = (uint32_t*)dwt.p;
-    launch_pack_bf16(st, dw.f(), rows, k, wt);
-    launch_mm_exact(st, BF16, dx.f(), m, k, wt, nullptr, rows, dyref.f());
+    launch_pack_bf16(st, dw, rows, k, wt);
+    launch_mm_exact(st, BF16, dx, m, k, wt, nullptr, rows, dyref);
     // every alpha's product first, then their error sums side by side
     for (int step = 0; step < kSteps; step++) {
-        const float *sv = dsc.f() + (size_t)step * 2 * k, *imp = sv + k;
-        launch_quantize(st, kind, rows, k, dw.f(), sv, imp, nullptr, wt, ds.f());
-        launch_scale_cols(st, dx.f(), (int64_t)mk, k, sv, dxs.f());
-        launch_mm_exact(st, kind, dxs.f(), m, k, wt, ds.f(), rows, dy.f() + (size_t)step * ny);
+        const float *sv = dsc + (size_t)step * 2 * k, *imp = sv + k;
+        launch_quantize(st, kind, rows, k, dw, sv, imp, nullptr, wt, ds);
+        launch_scale_cols(st, dx, (int64_t)mk, k, sv, dxs);
+        launch_mm_exact(st, kind, dxs, m, k, wt, ds, rows, dy + (size_t)step * ny);
     }
-    launch_sq_err(st, dy.f(), (int64_t)ny, kSteps, dyref.f(), (int64_t)ny, dwork.p, (double*)derr.p);
+    launch_sq_err(st, dy, (int64_t)ny, kSteps, dyref, (int64_t)ny, dwork, derr);
     HIPCHK(hipGetLastError());
     double errs[kSteps];
-    HIPCHK(hipMemcpyAsync(errs, derr.p, sizeof(errs), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync(errs, derr, sizeof(errs), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     double best = INFINITY, plain = errs[0];
     int best_step = 0;
@@ -2025,12 +2245,10 @@ int fg_awq_search(fg_ctx* ctx, int32_t kind, int32_t rows, int32_t k, const floa
             best = errs[step];
             best_step = step;
         }
-    const float* bs = dsc.f() + (size_t)best_step * 2 * k;
-    launch_quantize(st, kind, rows, k, dw.f(), bs, bs + k, dq.u8(), nullptr, ds.f());
+    const float* bs = dsc + (size_t)best_step * 2 * k;
+    launch_quantize(st, kind, rows, k, dw, bs, bs + k, dq, nullptr, ds);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(q, dq.p, qb, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(s, ds.p, sn * 4, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    if ((rc = copy_host(ctx, q, dq, qb, false)) || (rc = copy_host(ctx, s, ds, sn * 4, false))) return rc;
     std::memcpy(scales, scales_of(best_step), (size_t)k * 4);
     choice->alpha = (float)best_step / 10.0f;
     choice->_pad = 0;

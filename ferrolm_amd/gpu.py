@@ -347,7 +347,7 @@ def forward(ctx: Context, model: Model, kv: KvCache, chunks, logits: bool = True
         arr[i] = FgChunk(ptr(tok, u32p), len(tok), pos, ptr(blocks, u32p), len(blocks), mode)
         rows += len(tok) if mode == LOGITS_ALL else (1 if mode == LOGITS_LAST and len(tok) else 0)
         t += len(tok)
-    lg = np.zeros((rows, model.cfg.vocab), np.float32) if logits else None
+    lg = np.empty((rows, model.cfg.vocab), np.float32) if logits else None
     am = np.zeros(rows, np.uint32)
     hid = np.zeros((model.cfg.layers + 1, t, model.cfg.hidden), np.float32) if hidden else None
     nrows = C.c_int32(0)
@@ -566,8 +566,8 @@ class Mat:
 
 
 def _qmatrix_buffers(kind: int, rows: int, cols: int):
-    q = np.zeros(rows * cols // (1 if kind == INT8 else 2), np.uint8)
-    s = np.zeros(rows * cols // 32, np.float32)
+    q = np.empty(rows * cols // (1 if kind == INT8 else 2), np.uint8)
+    s = np.empty(rows * cols // 32, np.float32)
     return q, s
 
 

@@ -44,3 +44,30 @@ def test_search_errors_across_chunks(ctx, rows, m):
     assert got[1:4] == tuple(want[1:4])
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[4].q, want[4].q)
     assert np.array_equal(got[4].s, want[4].s)
+
+
+@pytest.mark.parametrize("kind", [INT8, INT4], ids=["int8", "int4"])
+@pytest.mark.parametrize("rows,cols", [(2016, 2048), (2048, 2048), (2080, 2080), (160, 32768), (160, 32800)])
+def test_large_matrices_in_panels(ctx, kind, rows, cols):
+    """Copied whole (under 16 MB, or panels over 4 MB) or through staging slots of
+    whole panels, the last one short: a panel's codes and scales are those it
+    has on its own."""
+    rng = np.random.default_rng(rows)
+    w = (0.02 * rng.standard_normal((rows, cols))).astype(np.float32)
+    imp = rng.random(cols).astype(np.float32)
+    for weight in (None, imp):
+        got = gpu.quantize(ctx, kind, w, weight)
+        parts = [gpu.quantize(ctx, kind, w[r : r + 32], weight) for r in range(0, rows, 32)]
+        assert np.array_equal(got.q.ravel(), np.concatenate([p.q.ravel() for p in parts]))
+        assert np.array_equal(got.s.ravel(), np.concatenate([p.s.ravel() for p in parts]))
+
+
+def test_search_copies_a_large_matrix(ctx):
+    """17 MB of weights in five slots, the last one short."""
+    rng = np.random.default_rng(3)
+    w = (0.02 * rng.standard_normal((2080, 2080))).astype(np.float32)
+    cal = rng.standard_normal((4, 2080)).astype(np.float32)
+    got, want = gpu.awq_search(ctx, INT8, w, cal), oracle.awq_search(INT8, w, cal)
+    assert got[1:4] == tuple(want[1:4])
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[4].q, want[4].q)
+    assert np.array_equal(got[4].s, want[4].s)
