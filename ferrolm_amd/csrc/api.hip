@@ -534,26 +534,42 @@ static int build_plan(const fg_config& c, const fg_kv& kv, int max_pos, const Ch
     if (c.head_dim == 64 && w1 * c.kv_heads >= kTwoSubSpanItems && maxq > 4) P.ns = 128 / span1;
     P.maxq = maxq;
     const int span = span1 * P.ns;
-    // Long chunks at hd 64 and 128 take the flash items (rf rows each, split into
-    // parts of at most kFlashPart positions: on the 1.7B shape's 1024-token
-    // prefill 15.7 ms unsplit, 15.5 at 512, 15.3 at 256) when there are at least
-    // 256 rows and enough parts to spread over the CUs.
+    // Long chunks at hd 64 and 128 take the flash items (rf rows each, split into parts of at most
+    // kFlashPart positions). Where every chunk fills an item: from 64 rows and 96 parts x kv heads
+    // (hd 64; 256 at hd 128) on, the parts halved down to 64 positions until there are kFlashParts.
+    // us per prefill with span items -> flash items, 1.7B int4: 96 rows (96 parts) 2187 -> 2179, 160
+    // 2806 -> 2768, 512 in 384 parts 5793 -> 5654, in 640 5509, 1024 rows 9947 -> 9404; 135M: 256 rows
+    // (97 parts) 1719 -> 1680, 400 1939 -> 1849, 777 2790 -> 2340 in 423 parts, 2468 in 750; 8B (hd
+    // 128): 64 rows (32 parts) 1380 -> 1423, 160 (144) 2142 -> 2175, 256 (320) 2883 -> 2862, 1024
+    // 8864 -> 8590. Batches with shorter chunks leave most of an item's 64 queries empty: from 256
+    // rows and parts on.
     const int rf = 2 * (attn_qmax(c.head_dim) / group);
     const int fblk = kFlashBlock(c.head_dim);
+    int fpart = kFlashPart;
     auto flash_parts = [&](int L) {
-        const int nb = (L + fblk - 1) / fblk, per = kFlashPart / fblk;
+        const int nb = (L + fblk - 1) / fblk, per = fpart / fblk;
         return (nb + per - 1) / per;
     };
-    {
-        int64_t parts = 0, rows = 0;
-        for (int ci = 0; ci < nch; ci++)
-            if (ch[ci].n > 0) {
-                rows += ch[ci].n;
-                if (rf >= 2)
-                    for (int r0 = 0; r0 < ch[ci].n; r0 += rf)
-                        parts += flash_parts(ch[ci].pos + r0 + std::min(rf, ch[ci].n - r0));
-            }
-        P.flash = (c.head_dim == 64 || c.head_dim == 128) && rf >= 2 && rows >= 256 && parts * c.kv_heads >= 256;
+    if ((c.head_dim == 64 || c.head_dim == 128) && rf >= 2) {
+        int64_t rows = 0;
+        bool fill = true;
+        for (int ci = 0; ci < nch; ci++) {
+            rows += std::max(ch[ci].n, 0);
+            fill = fill && (ch[ci].n <= 0 || ch[ci].n >= rf);
+        }
+        auto count = [&] {
+            int64_t parts = 0;
+            for (int ci = 0; ci < nch; ci++)
+                for (int r0 = 0; r0 < ch[ci].n; r0 += rf)
+                    parts += flash_parts(ch[ci].pos + r0 + std::min(rf, ch[ci].n - r0));
+            return parts * c.kv_heads;
+        };
+        int64_t parts = rows >= (fill ? 64 : 256) ? count() : 0;
+        while (fill && parts > 0 && parts < kFlashParts && fpart > 64) {
+            fpart /= 2;
+            parts = count();
+        }
+        P.flash = parts >= (fill && c.head_dim == 64 ? 96 : 256);
         if (P.flash) P.ns = 1;
     }
     for (int ci = 0; ci < nch; ci++) {

@@ -256,9 +256,12 @@ constexpr int kAttnMfmaQueries = 16;
 // at 32 sequences, 3 x 576 slots, draft 4886 -> 4795 us per step; the cfg2
 // draft's 3 x 32 +12 us per step; the cfg2 verify's 32 x 32 unchanged).
 constexpr int kAttnDecWorkgroups = 1024;
-// Positions per block of the flash attention items, and per part of an item.
+// Positions per block of the flash attention items, the most per part of an item, and the
+// workgroups below which a launch of full items takes shorter parts (one and a half a CU; more
+// parts than it takes to get there cost more in the merge than they gain).
 constexpr int kFlashBlock(int hd) { return hd >= 128 ? 32 : 64; }
 constexpr int kFlashPart = 256;
+constexpr int kFlashParts = 400;
 
 // ---------------------------------------------------------------------------
 // Sampling (sampling.hip). A row's distribution is stored in the reference's

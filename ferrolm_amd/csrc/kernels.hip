@@ -2103,22 +2103,29 @@ __global__ __launch_bounds__(256, MINW) void k_attn(AttnArgs a) {
 // an item being up to 2 * (32 / G) consecutive rows of one chunk (at most 64
 // queries, G query heads per kv head). The workgroup walks every position the
 // item's last row sees (or a part of them) in blocks of P (64 at hd 64, 32 at
-// hd 128, so that two workgroups fit a CU's LDS): keys (rotated when new) and values go
-// through LDS, shared by the four waves; each wave owns 16 queries and keeps
-// their online softmax (running max and sum, weighted values) in registers,
-// scores and weighted values on f32 MFMA. The next block's loads are issued
-// before the current one is scored. The item's two row halves write their
-// partials (max score, sum of exponentials, weighted values) to the work-item
-// slots their record names: the layout the span merge reads, one span per part.
+// hd 128): keys (rotated when new) and values go through LDS, shared by the four
+// waves; each wave owns 16 queries. The next block's loads are issued before the
+// current one is scored. The item's two row halves write their partials (max
+// score, sum of exponentials, weighted values) to the work-item slots their
+// record names: the layout the span merge reads, one span per part.
+//
+// Bound: the f32 MFMAs (32 cycles each, 29 us of the 1.7B shape's 1024-token
+// prefill layer). So that little else is in their way, both products are taken
+// transposed, with the order of the inner index chosen so that operands come
+// as they lie: S^T = K Q^T leaves lane (kk, c) (lane = 16 kk + c) with query
+// c's scores of positions 16 t + 4 kk + r in register r of tile t, which is
+// where O^T = V^T P^T wants them, so the probabilities never leave their
+// registers, a query's maximum is two shuffles, and its running max, sum and
+// rescaling factor are the lane's own; keys and values come from LDS four
+// floats at a read, and the queries stay in registers. 1.7B layer, 1024 tokens:
+// 91.9 -> 69.1 us; 135M layer, 777 tokens: 33 (span items) -> 18.5 us. Three
+// workgroups a CU (four spill, two are no faster).
 template <int HD, int P>
-__global__ __launch_bounds__(256, 2) void k_attn_flash(AttnArgs a) {
-    constexpr int HALF = HD / 2, QM = 32, NTD = HD / 16;
+__global__ __launch_bounds__(256, 3) void k_attn_flash(AttnArgs a) {
+    constexpr int HALF = HD / 2, QM = 32, NS = HD / 16, NH = HD / 64, NT = P / 16;
     static_assert(P % 16 == 0 && 64 % P == 0, "blocks of whole 16-position MFMA tiles");
     __shared__ __align__(16) float ks[P][HD + 4];
-    __shared__ __align__(16) float vs[P][vstride(HD)];
-    __shared__ __align__(16) float qs[64][HD + 4];
-    __shared__ __align__(16) float pw[4][16][P + 4];
-    __shared__ int lim[64];
+    __shared__ __align__(16) float vs[P][HD];
 
     const int h = blockIdx.x, fi = blockIdx.y;
     const int4* rec = (const int4*)(a.wrec + (size_t)fi * 16);
@@ -2129,11 +2136,14 @@ __global__ __launch_bounds__(256, 2) void k_attn_flash(AttnArgs a) {
     if (nrows == 0) return;  // an unused slot of the launch's capacity
     const int G = a.nh / a.nkv, Q = nrows * G, RQ = QM / G;
     const int qd = a.nh * HD;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kk = lane >> 4, c16 = lane & 15;
     const int32_t* bt = a.btab + boff;
     const int pos_of_row0 = cpos0 + row0 - crow0;
-    for (int q = tid; q < 64; q += 256) lim[q] = q < Q ? pos_of_row0 + q / G : -1;
+    // the lane's query, the last position it sees, and the last any of the wave's does
+    const int q = wave * 16 + c16, qr = q < Q ? q / G : 0;
+    const int lq = q < Q ? pos_of_row0 + qr : -1;
+    const int lw = Q > wave * 16 ? pos_of_row0 + (min(Q, wave * 16 + 16) - 1) / G : -1;
 
     // position p's key (col 0) or value (col HD * nkv): the cache, or this chunk's q/k/v rows
     auto src_of = [&](int p, int col) -> const float* {
@@ -2148,8 +2158,8 @@ __global__ __launch_bounds__(256, 2) void k_attn_flash(AttnArgs a) {
         for (int it = 0; it < KIT; it++) {
             const int i = tid + it * 256, d = (i % (HALF / 4)) * 4, p = min(b0 + i / (HALF / 4), L - 1);
             const float* kp = src_of(p, 0);
-            ku[it] = ld_nt_f4(kp + d);
-            kw[it] = ld_nt_f4(kp + d + HALF);
+            ku[it] = *(const float4*)(kp + d);
+            kw[it] = *(const float4*)(kp + d + HALF);
             const int pr = max(p, cpos0);
             kcs[it] = *(const float4*)(a.cos_t + (size_t)pr * HALF + d);
             ksn[it] = *(const float4*)(a.sin_t + (size_t)pr * HALF + d);
@@ -2157,151 +2167,158 @@ __global__ __launch_bounds__(256, 2) void k_attn_flash(AttnArgs a) {
 #pragma unroll
         for (int it = 0; it < VIT; it++) {
             const int i = tid + it * 256, d = (i % (HD / 4)) * 4, p = min(b0 + i / (HD / 4), L - 1);
-            vv[it] = ld_nt_f4(src_of(p, a.nkv * HD) + d);
+            vv[it] = *(const float4*)(src_of(p, a.nkv * HD) + d);
         }
     };
+    // (a, b) rotated by (cos, sin): the first half's element, then the second's
+    auto rot1 = [](float x, float y, float c, float s) { return __fadd_rn(__fmul_rn(x, c), __fmul_rn(-y, s)); };
+    auto rot2 = [](float x, float y, float c, float s) { return __fadd_rn(__fmul_rn(y, c), __fmul_rn(x, s)); };
     load_blk(p0);
-    // the queries, rotated; rows past Q are zero
-    for (int i = tid; i < 64 * (HALF / 4); i += 256) {
-        const int q = i / (HALF / 4), d = (i % (HALF / 4)) * 4;
-        float r1v[4] = {0, 0, 0, 0}, r2v[4] = {0, 0, 0, 0};
-        if (q < Q) {
-            const int r = q / G, j = q % G, pos = pos_of_row0 + r;
-            const float* src = a.qkv + (size_t)(row0 + r) * a.ld + (size_t)(h * G + j) * HD;
-            const float4 x1 = *(const float4*)(src + d), x2 = *(const float4*)(src + d + HALF);
+    // the lane's query, rotated: inputs 16 s + 4 kk + e
+    float qv[NS][4];
+    {
+        const int pos = pos_of_row0 + qr;
+        const float* src = a.qkv + (size_t)(row0 + qr) * a.ld + (size_t)(h * G + (q < Q ? q % G : 0)) * HD;
+#pragma unroll
+        for (int s = 0; s < NS / 2; s++) {
+            const int d = 16 * s + 4 * kk;
+            const float4 x = *(const float4*)(src + d), y = *(const float4*)(src + d + HALF);
             const float4 c = *(const float4*)(a.cos_t + (size_t)pos * HALF + d);
-            const float4 sn = *(const float4*)(a.sin_t + (size_t)pos * HALF + d);
-            const float a1[4] = {x1.x, x1.y, x1.z, x1.w}, a2[4] = {x2.x, x2.y, x2.z, x2.w};
-            const float cc[4] = {c.x, c.y, c.z, c.w}, ss[4] = {sn.x, sn.y, sn.z, sn.w};
+            const float4 n = *(const float4*)(a.sin_t + (size_t)pos * HALF + d);
+            const float xs[4] = {x.x, x.y, x.z, x.w}, ys[4] = {y.x, y.y, y.z, y.w};
+            const float cs[4] = {c.x, c.y, c.z, c.w}, ns[4] = {n.x, n.y, n.z, n.w};
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                r1v[e] = __fadd_rn(__fmul_rn(a1[e], cc[e]), __fmul_rn(-a2[e], ss[e]));
-                r2v[e] = __fadd_rn(__fmul_rn(a2[e], cc[e]), __fmul_rn(a1[e], ss[e]));
+                qv[s][e] = rot1(xs[e], ys[e], cs[e], ns[e]);
+                qv[s + NS / 2][e] = rot2(xs[e], ys[e], cs[e], ns[e]);
             }
-        }
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            qs[q][d + e] = r1v[e];
-            qs[q][d + HALF + e] = r2v[e];
         }
     }
 
-    float mrow[4], lrow[4];
-    f32x4 oc[NTD];
+    float mrow = -INFINITY, lrow = 0.0f;  // lrow: of the lane's own positions
+    f32x4 oc[NH][4];  // values 64 hh + 16 kk + 4 r + j of the lane's query in oc[hh][j][r]
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-        mrow[r] = -INFINITY;
-        lrow[r] = 0.0f;
-    }
+    for (int hh = 0; hh < NH; hh++)
 #pragma unroll
-    for (int j = 0; j < NTD; j++) oc[j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+        for (int j = 0; j < 4; j++) oc[hh][j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
     const int nblk = (L - p0 + P - 1) / P;
-    const int q0 = wave * 16;
     for (int b = 0; b < nblk; b++) {
         const int b0 = p0 + b * P;
-        if (b > 0) __syncthreads();  // the previous block's readers of ks, vs and pw are done
+        if (b > 0) __syncthreads();  // the previous block's readers of ks and vs are done
 #pragma unroll
         for (int it = 0; it < KIT; it++) {
             const int i = tid + it * 256, o = i / (HALF / 4), d = (i % (HALF / 4)) * 4, p = b0 + o;
-            const float a1[4] = {ku[it].x, ku[it].y, ku[it].z, ku[it].w};
-            const float a2[4] = {kw[it].x, kw[it].y, kw[it].z, kw[it].w};
-            const float cc[4] = {kcs[it].x, kcs[it].y, kcs[it].z, kcs[it].w};
-            const float ss[4] = {ksn[it].x, ksn[it].y, ksn[it].z, ksn[it].w};
+            const float xs[4] = {ku[it].x, ku[it].y, ku[it].z, ku[it].w};
+            const float ys[4] = {kw[it].x, kw[it].y, kw[it].z, kw[it].w};
+            const float cs[4] = {kcs[it].x, kcs[it].y, kcs[it].z, kcs[it].w};
+            const float ns[4] = {ksn[it].x, ksn[it].y, ksn[it].z, ksn[it].w};
             const bool live = p < L, rot = live && p >= cpos0;
+            float x[4], y[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const float x1 = rot ? __fadd_rn(__fmul_rn(a1[e], cc[e]), __fmul_rn(-a2[e], ss[e])) : a1[e];
-                const float x2 = rot ? __fadd_rn(__fmul_rn(a2[e], cc[e]), __fmul_rn(a1[e], ss[e])) : a2[e];
-                ks[o][d + e] = live ? x1 : 0.0f;
-                ks[o][d + HALF + e] = live ? x2 : 0.0f;
+                x[e] = rot ? rot1(xs[e], ys[e], cs[e], ns[e]) : live ? xs[e] : 0.0f;
+                y[e] = rot ? rot2(xs[e], ys[e], cs[e], ns[e]) : live ? ys[e] : 0.0f;
             }
+            *(float4*)&ks[o][d] = make_float4(x[0], x[1], x[2], x[3]);
+            *(float4*)&ks[o][d + HALF] = make_float4(y[0], y[1], y[2], y[3]);
         }
 #pragma unroll
         for (int it = 0; it < VIT; it++) {
             const int i = tid + it * 256, o = i / (HD / 4), d = (i % (HD / 4)) * 4;
             const bool live = b0 + o < L;
-            *(float4*)&vs[o][vcol<HD>(o, d)] = make_float4(live ? vv[it].x : 0.0f, live ? vv[it].y : 0.0f,
+            *(float4*)&vs[o][d] = make_float4(live ? vv[it].x : 0.0f, live ? vv[it].y : 0.0f,
                                               live ? vv[it].z : 0.0f, live ? vv[it].w : 0.0f);
         }
         __syncthreads();
         if (b + 1 < nblk) load_blk(b0 + P);
         // this item's new rows in the block go to the cache
         {
-            const int n0 = max(b0, pos_of_row0), n1 = min(b0 + P, pos_of_row0 + nrows);
-            for (int i = tid; i < (n1 - n0) * HD; i += 256) {
-                const int p = n0 + i / HD, d = i % HD, o = p - b0;
+            const int n0 = max(b0, pos_of_row0), n1 = min(min(b0 + P, L), pos_of_row0 + nrows);
+            for (int i = tid; i < (n1 - n0) * (HD / 4); i += 256) {
+                const int p = n0 + i / (HD / 4), d = (i % (HD / 4)) * 4, o = p - b0;
                 const size_t at = (((size_t)(uint32_t)bt[p >> 4] * a.nkv + h) * 16 + (p & 15)) * HD + d;
-                a.kc[at] = ks[o][d];
-                a.vc[at] = vs[o][vcol<HD>(o, d)];
+                *(float4*)(a.kc + at) = *(const float4*)&ks[o][d];
+                *(float4*)(a.vc + at) = *(const float4*)&vs[o][d];
             }
         }
-        // the wave's 16 x 64 scores (v_mfma_f32_16x16x4f32: A[i][k] in lane i + 16k,
-        // B[k][j] in lane j + 16k, D[4(l/16) + r][l%16] in register r of lane l)
-        f32x4 sc[P / 16];
+        if (lw < b0) continue;  // no query of the wave sees the block
+        // scores (v_mfma_f32_16x16x4f32: A[i][k] in lane i + 16k, B[k][j] in lane
+        // j + 16k, D[4(l/16) + r][l%16] in register r of lane l)
+        f32x4 sc[NT];
 #pragma unroll
-        for (int nt = 0; nt < P / 16; nt++) {
-            const float* qa = &qs[q0 + c16][kk];
-            const float* kb = &ks[nt * 16 + c16][kk];
+        for (int t = 0; t < NT; t++) {
             f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int d0 = 0; d0 < HD; d0 += 4) c = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[d0], kb[d0], c, 0, 0, 0);
-            sc[nt] = c;
+            for (int s = 0; s < NS; s++) {
+                const float4 k = *(const float4*)&ks[t * 16 + c16][16 * s + 4 * kk];
+                c = __builtin_amdgcn_mfma_f32_16x16x4f32(k.x, qv[s][0], c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x4f32(k.y, qv[s][1], c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x4f32(k.z, qv[s][2], c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x4f32(k.w, qv[s][3], c, 0, 0, 0);
+            }
+            sc[t] = c;
         }
-        // online softmax of each of the lane's four query rows; a row's 64 scores
-        // sit in the 16 lanes of its lane group, four per lane
+        // online softmax of the lane's query
+        float mx = -INFINITY;
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int lq = lim[q0 + 4 * kk + r];
-            float mx = -INFINITY;
+        for (int t = 0; t < NT; t++)
 #pragma unroll
-            for (int nt = 0; nt < P / 16; nt++) {
-                const float v = b0 + nt * 16 + c16 <= lq ? sc[nt][r] * a.scale : -INFINITY;
-                sc[nt][r] = v;
+            for (int r = 0; r < 4; r++) {
+                const float v = b0 + t * 16 + 4 * kk + r <= lq ? sc[t][r] * a.scale : -INFINITY;
+                sc[t][r] = v;
                 mx = fmaxf(mx, v);
             }
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float mn = fmaxf(mrow, mx);
+        const float f = mrow == -INFINITY ? 0.0f : dev_exp(mrow - mn);
+        float sum = 0.0f;
 #pragma unroll
-            for (int off = 8; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 16));
-            const float mn = fmaxf(mrow[r], mx);
-            const float f = mrow[r] == -INFINITY ? 0.0f : dev_exp(mrow[r] - mn);
-            float sum = 0.0f;
+        for (int t = 0; t < NT; t++)
 #pragma unroll
-            for (int nt = 0; nt < P / 16; nt++) {
-                const float e = sc[nt][r] == -INFINITY ? 0.0f : dev_exp(sc[nt][r] - mn);
-                pw[wave][4 * kk + r][nt * 16 + c16] = e;
+            for (int r = 0; r < 4; r++) {
+                const float e = sc[t][r] == -INFINITY ? 0.0f : dev_exp(sc[t][r] - mn);
+                sc[t][r] = e;
                 sum += e;
             }
+        lrow = fmaf(lrow, f, sum);
+        mrow = mn;
 #pragma unroll
-            for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 16);
-            lrow[r] = fmaf(lrow[r], f, sum);
-            mrow[r] = mn;
+        for (int hh = 0; hh < NH; hh++)
 #pragma unroll
-            for (int j = 0; j < NTD; j++) oc[j][r] *= f;
-        }
-        __syncthreads();  // pw rows are read across the wave's lanes
-        // weighted values: O += P V over the block's 64 positions
+            for (int j = 0; j < 4; j++)
 #pragma unroll
-        for (int j = 0; j < NTD; j++) {
-            const float* pa = &pw[wave][c16][kk];
-            const float* vb = &vs[kk][vcol<HD>(kk, j * 16 + c16)];  // rows kk + k0: k0 % 4 == 0
+                for (int r = 0; r < 4; r++) oc[hh][j][r] *= f;
+        // weighted values over the block's positions
 #pragma unroll
-            for (int k0 = 0; k0 < P; k0 += 4)
-                oc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[k0], vb[k0 * vstride(HD)], oc[j], 0, 0, 0);
-        }
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int hh = 0; hh < NH; hh++) {
+                    const float4 v = *(const float4*)&vs[t * 16 + 4 * kk + r][64 * hh + 4 * c16];
+                    oc[hh][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.x, sc[t][r], oc[hh][0], 0, 0, 0);
+                    oc[hh][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.y, sc[t][r], oc[hh][1], 0, 0, 0);
+                    oc[hh][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.z, sc[t][r], oc[hh][2], 0, 0, 0);
+                    oc[hh][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.w, sc[t][r], oc[hh][3], 0, 0, 0);
+                }
     }
+    lrow += __shfl_xor(lrow, 16);
+    lrow += __shfl_xor(lrow, 32);
     // the partials of the item's two row halves
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int q = q0 + 4 * kk + r;
-        if (q < Q) {
-            const int half = q / G >= RQ ? 1 : 0;
-            float* pq = a.part + (((size_t)(half ? slot1 : slot0) * a.nkv + h) * QM + (q - half * RQ * G)) * (HD + 4);
-            if (c16 == 0) {
-                pq[0] = mrow[r];
-                pq[1] = lrow[r];
-            }
-#pragma unroll
-            for (int j = 0; j < NTD; j++) pq[4 + j * 16 + c16] = oc[j][r];
+    if (q < Q) {
+        const int half = qr >= RQ ? 1 : 0;
+        float* pq = a.part + (((size_t)(half ? slot1 : slot0) * a.nkv + h) * QM + (q - half * RQ * G)) * (HD + 4);
+        if (kk == 0) {
+            pq[0] = mrow;
+            pq[1] = lrow;
         }
+#pragma unroll
+        for (int hh = 0; hh < NH; hh++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                *(float4*)(pq + 4 + 64 * hh + 16 * kk + 4 * r) =
+                    make_float4(oc[hh][0][r], oc[hh][1][r], oc[hh][2][r], oc[hh][3][r]);
     }
 }
 
