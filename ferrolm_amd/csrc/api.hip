@@ -74,7 +74,7 @@ struct Carver {
 // ---------------------------------------------------------------------------
 // Handles
 // ---------------------------------------------------------------------------
-// Staging of large host copies (copy_host, quantize_staged): kSlots slots, each a pinned and a
+// Staging of large host copies (copy_host, fg_quantize): kSlots slots, each a pinned and a
 // device region for kSlotIn bytes of input and kSlotOut of output; a worker thread t owns slots
 // t * kSlotsEach ... and streams[t]. Made by the first call that wants it, freed with
 // the context.
