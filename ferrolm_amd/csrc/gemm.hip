@@ -45,10 +45,10 @@ int launch_mm(hipStream_t st, int epi, const DMat& w, const GemvArgs& a, hipEven
             tiles = n;
         }
     }
-    // k_gemm splits K finer and wins where the tiles leave CUs idle: 6144 x 2048 at 160 rows (240 tiles
-    // of two row tiles) 22.4 against 21.9 us, at 192 (192 of three) 32.2 against 25.3; 2048 x 8192 at 256
-    // (128) 42 against 59, at 320 (160) 69 against 61; and on short K with two row tiles (960 x 576 at
-    // 1024 rows 14.5 against 16.2).
+    // k_gemm splits K finer and wins where the tiles leave CUs idle. Its time, then the tiles', in us:
+    // 2048 x 8192 at 256 rows (128 tiles) 42 against 59, at 320 (160) 69 against 61; 6144 x 2048 at 160
+    // (240 of two row tiles) even, 22.4 against 21.9, at 192 (192 of three) 32.2 against 25.3; and on
+    // short K with two row tiles 960 x 576 at 1024 rows 14.5 against 16.2.
     if (kTiles[cfg].rt == 2 ? tiles < 150 || a.m < 256 || a.KB < 32 : tiles < 180) return 0;
     if (w.kind == INT4)
         run_mm<INT4>(st, epi, cfg, a, e0, e1);
