@@ -382,7 +382,7 @@ def measure_batched(a, wl, ctx, target, draft, B: int, steps: int, warmup: int) 
             roofline = {"bound": "mfma", "achieved": round(ach, 2), "peak": 2500.0, "unit": "TFLOP/s",
                         "frac": round(ach / 2500.0, 5), "mfma_issue_frac": round(2 * ach / 2500.0, 5),
                         "traffic": None,
-                        "kernel": f"k_gemm {dom['kind']} weights, bf16 MFMA (target verify GEMMs, {B * (k + 1)} rows)",
+                        "kernel": f"k_gemm / k_mm {dom['kind']} weights, bf16 MFMA (target verify GEMMs, {B * (k + 1)} rows)",
                         "flops_per_launch": round(dom["flops"] / dom["launches"]),
                         "us_per_launch": round(dom["us"] / dom["launches"], 3), "launches": dom["launches"]}
     rec = {"workload": f"{wl.name}: {KIND_NAMES[wl.target_kind]} target ({cfg.layers} layers, hidden {cfg.hidden}) "
