@@ -1284,11 +1284,17 @@ int fg_ctx_create(int device, fg_ctx** out) {
         return fail(FG_E_DEVICE, "stream creation failed");
     }
     for (auto& e : c->ev) HIPCHK(hipEventCreate(&e));
-    if (hipMalloc((void**)&c->gcnt, kGemvSplitGroups * 32 * sizeof(unsigned)) != hipSuccess) {
+    const size_t counters = kGemvSplitGroups * 32 * sizeof(unsigned);
+    if (hipMalloc((void**)&c->gcnt, counters) != hipSuccess) {
         fg_ctx_destroy(c);
         return fail(FG_E_NOMEM, "counter allocation failed");
     }
-    HIPCHK(hipMemset(c->gcnt, 0, kGemvSplitGroups * 32 * sizeof(unsigned)));
+    // cleared on the context's stream: it does not wait for the default stream, so a clear queued
+    // there could still run between two arrivals on a counter, and that output would never be finished
+    if (hipMemsetAsync(c->gcnt, 0, counters, c->stream) != hipSuccess) {
+        fg_ctx_destroy(c);
+        return fail(FG_E_DEVICE, "counter clear failed");
+    }
     c->scratch = scratch_address(device);
     const char* ng = std::getenv("FERRO_NO_GRAPH");
     c->graphs = !(ng && ng[0] == '1');
@@ -1924,7 +1930,7 @@ int fg_stamps_reset(fg_ctx* ctx) {
     if (!ctx) return fail(FG_E_ARG, "null ctx");
     HIPCHK(hipSetDevice(ctx->device));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (stamps_clear()) return fail(FG_E_ARG, "this library was built without stamps (python -m ferrolm_amd.build --stamps)");
+    if (stamps_clear(ctx->stream)) return fail(FG_E_ARG, "this library was built without stamps (python -m ferrolm_amd.build --stamps)");
     return 0;
 }
 

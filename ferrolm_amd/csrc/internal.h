@@ -334,6 +334,6 @@ void launch_sq_err(hipStream_t st, const float* y, int64_t ystride, int count, c
 // `slots` slots; both return -1 in a library built without stamps.
 constexpr int kStampSlots = 1024, kStampWgs = 1024;
 int stamps_read(uint64_t* out, int slots);
-int stamps_clear();
+int stamps_clear(hipStream_t st);
 
 }  // namespace fg

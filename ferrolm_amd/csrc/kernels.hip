@@ -2763,14 +2763,14 @@ int stamps_read(uint64_t* out, int slots) {
     if (slots < 0 || slots > kStampSlots) return -1;
     return hipMemcpyFromSymbol(out, HIP_SYMBOL(g_stamps), (size_t)slots * kStampWgs * 2 * 8) == hipSuccess ? 0 : -1;
 }
-int stamps_clear() {
+int stamps_clear(hipStream_t st) {
     void* p = nullptr;
     if (hipGetSymbolAddress(&p, HIP_SYMBOL(g_stamps)) != hipSuccess) return -1;
-    return hipMemset(p, 0, sizeof(g_stamps)) == hipSuccess ? 0 : -1;
+    return hipMemsetAsync(p, 0, sizeof(g_stamps), st) == hipSuccess ? 0 : -1;
 }
 #else
 int stamps_read(uint64_t*, int) { return -1; }
-int stamps_clear() { return -1; }
+int stamps_clear(hipStream_t) { return -1; }
 #endif
 
 int launch_attention(hipStream_t st, const AttnArgs& a, int m, int consumer_kind, Pieces& out) {

@@ -1,0 +1,53 @@
+"""The library's host code on a HIP runtime of the CPU (fake_hip.cpp) that runs
+queued work as late as a device may: memory is clear before a handle to it is
+returned."""
+import os
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+
+# the fake's names come first in the library's symbol lookup
+PRELUDE = """
+import ctypes, sys
+import numpy as np
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+from ferrolm_amd import gpu, host
+from ferrolm_amd.weights import INT4, INT8, Config
+fail = lambda name, nth=1: fake.fake_fail(name.encode(), nth)
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    """Runs code after PRELUDE in a process of its own, which has no other HIP runtime to find."""
+    lib = tmp_path_factory.mktemp("hip") / "libfake_hip.so"
+    subprocess.run(["g++", "-std=c++17", "-O2", "-shared", "-fPIC", "-o", str(lib),
+                    str(ROOT / "tests" / "fake_hip.cpp"), "-ldl", "-lpthread"], check=True, timeout=120)
+
+    def go(code):
+        env = dict(os.environ, FERRO_GPU_LIB=str(ROOT / "ferrolm_amd" / "libferro_gpu.so"))
+        r = subprocess.run([sys.executable, "-c", PRELUDE + code, str(lib)], cwd=ROOT, env=env, capture_output=True,
+                           text=True, timeout=300)
+        assert r.returncode == 0, r.stdout + r.stderr
+
+    return go
+
+
+def test_a_new_context_waits_for_its_counters_to_be_clear(run):
+    """The split products' arrival counters: a clear left on the default stream would run beside the first
+    launches on the context's stream, which does not wait for it."""
+    run("""
+c = gpu.Context(0)
+assert fake.fake_pending_default() == 0
+c.close()
+""")
+
+
+def test_no_clear_is_left_on_the_default_stream():
+    """No source of the library clears memory on the default stream, where no launch waits for it."""
+    for p in (ROOT / "ferrolm_amd" / "csrc").iterdir():
+        assert "hipMemset(" not in p.read_text(), p
