@@ -1448,10 +1448,11 @@ int fg_kv_create(fg_ctx* ctx, int32_t layers, int32_t kv_heads, int32_t head_dim
         fg_kv_destroy(kv);
         return fail(FG_E_NOMEM, "cache allocation failed");
     }
-    // cleared on the context's stream: it does not wait for the default stream, so a
-    // clear queued there could still be running over the first rows written here
+    // clear before the handle is returned: contexts' streams do not wait for each other or for the
+    // default stream, and any context on the device may write the cache's first rows
     if (hipMemsetAsync(kv->k, 0, bytes, ctx->stream) != hipSuccess ||
-        hipMemsetAsync(kv->v, 0, bytes, ctx->stream) != hipSuccess) {
+        hipMemsetAsync(kv->v, 0, bytes, ctx->stream) != hipSuccess ||
+        hipStreamSynchronize(ctx->stream) != hipSuccess) {
         fg_kv_destroy(kv);
         return fail(FG_E_DEVICE, "cache clear failed");
     }

@@ -154,7 +154,8 @@ int64_t fg_model_weight_bytes(const fg_model* m);
 /* KvCache::new (src/kv.rs:33-44): f32 keys and values for every layer in
  * the reference layout [layer][block][kv_head][block_size][head_dim].
  * block_size must be 16 (FG_E_ARG) and head_dim 16, 32, 64 or 128
- * (FG_E_SHAPE). */
+ * (FG_E_SHAPE). The cache is clear when the call returns: any context on
+ * the device may use it. */
 int fg_kv_create(fg_ctx* ctx, int32_t layers, int32_t kv_heads,
                  int32_t head_dim, int32_t block_size, int32_t blocks,
                  fg_kv** out);

@@ -1,7 +1,6 @@
-"""A new cache is clear before anything queued on its context touches it: rows
-written right after fg_kv_create stay (the clear of a large cache takes
-milliseconds on the device, and a clear on another stream could still be
-running over them)."""
+"""A new cache is clear when fg_kv_create returns: rows written right after it
+stay (the clear of a large cache takes milliseconds on the device, and one that
+was still running could go over them)."""
 import numpy as np
 import pytest
 

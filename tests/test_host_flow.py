@@ -51,3 +51,18 @@ def test_no_clear_is_left_on_the_default_stream():
     """No source of the library clears memory on the default stream, where no launch waits for it."""
     for p in (ROOT / "ferrolm_amd" / "csrc").iterdir():
         assert "hipMemset(" not in p.read_text(), p
+
+
+def test_a_new_cache_is_clear_for_every_context(run):
+    """Rows that a second context writes to a cache just made stay: the clear does not run after them."""
+    run("""
+a, b = gpu.Context(0), gpu.Context(0)
+cfg = Config(vocab=32, hidden=32, intermediate=32, layers=1, heads=2, kv_heads=2, head_dim=16)
+kv = gpu.KvCache(a, cfg, 4)
+k, v = np.random.default_rng(0).standard_normal((2, 4 * 16 * 2 * 16)).astype(np.float32)
+kv.ctx = b
+kv.set_layer(0, k, v)
+a.sync()
+got = kv.layer(0)
+assert np.array_equal(got[0], k) and np.array_equal(got[1], v)
+""")
