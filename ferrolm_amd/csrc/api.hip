@@ -23,7 +23,10 @@ namespace {
 
 thread_local std::string g_err;
 
+// The runtime keeps an error until it is read, and the check after the next call's launches would
+// report it again: it is read where it is returned.
 int fail(int code, const std::string& msg) {
+    if (code == FG_E_DEVICE || code == FG_E_NOMEM) (void)hipGetLastError();
     g_err = msg;
     return code;
 }
@@ -1125,7 +1128,6 @@ struct DevBuf {
 static int dev_alloc(DevBuf& b, size_t bytes) {
     if (hipMalloc(&b.p, std::max<size_t>(bytes, 256)) != hipSuccess) {
         b.p = nullptr;
-        (void)hipGetLastError();
         return fail(FG_E_NOMEM, "device allocation failed");
     }
     return 0;
@@ -1202,7 +1204,6 @@ static int staged(fg_ctx* c, size_t chunks, const I& issue, const F& finish) {
         if (x.joinable()) x.join();
     if (bad) {
         for (auto& x : g.streams) (void)hipStreamSynchronize(x);
-        (void)hipGetLastError();
         return fail(FG_E_DEVICE, "staged copy failed");
     }
     return 0;
@@ -1557,10 +1558,8 @@ int fg_forward_capture(fg_ctx* ctx, const fg_model* m, fg_kv* kv, const fg_chunk
     if ((rc = ensure(&ctx->ws, &ctx->ws_cap, need, ctx->stream, false))) return rc;
     layout_work(m, P, w, ctx->ws);
     float* cap = nullptr;
-    if (hipMalloc((void**)&cap, floats * 4) != hipSuccess) {
-        (void)hipGetLastError();
+    if (hipMalloc((void**)&cap, floats * 4) != hipSuccess)
         return fail(FG_E_NOMEM, "capture buffer of " + std::to_string(floats * 4) + " bytes");
-    }
     const int32_t* meta = (const int32_t*)ctx->dmeta;
     rc = run_forward(ctx, m, kv, P, meta, (const uint32_t*)(meta + P.o_tok), 1, w, nullptr, nullptr, nullptr, 0, 0,
                      nullptr, cap);

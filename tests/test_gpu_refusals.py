@@ -114,3 +114,12 @@ def test_cache_and_model_shape_refusals(ctx, setup):
     other = gpu.KvCache(ctx, replace(hm.cfg, kv_heads=hm.cfg.kv_heads * 2), 8)
     with pytest.raises(gpu.FgError, match="cache does not match the model"):
         gpu.forward(ctx, m, other, [([3, 4], 0, [0], gpu.LOGITS_LAST)])
+
+
+def test_a_refused_allocation_leaves_no_error_for_the_next_call(ctx, setup):
+    hm, m, kv = setup
+    want = gpu.forward(ctx, m, kv, [([3, 4, 5], 0, [2], gpu.LOGITS_LAST)])
+    with pytest.raises(gpu.FgError, match="cache allocation failed"):
+        gpu.KvCache(ctx, hm.cfg, 1 << 30)  # terabytes
+    got = gpu.forward(ctx, m, kv, [([3, 4, 5], 0, [2], gpu.LOGITS_LAST)])
+    assert np.array_equal(got.logits, want.logits)

@@ -1,6 +1,6 @@
 """The library's host code on a HIP runtime of the CPU (fake_hip.cpp) that runs
 queued work as late as a device may: memory is clear before a handle to it is
-returned."""
+returned, and a failed call leaves nothing behind."""
 import os
 import subprocess
 import sys
@@ -65,4 +65,22 @@ kv.set_layer(0, k, v)
 a.sync()
 got = kv.layer(0)
 assert np.array_equal(got[0], k) and np.array_equal(got[1], v)
+""")
+
+
+@pytest.mark.parametrize("failing", ["kv = gpu.KvCache(c, cfg, 1 << 30)", "fail('hipMemsetAsync'); gpu.KvCache(c, cfg, 4)",
+                                     "fail('hipStreamCreateWithFlags'); gpu.Context(0)",
+                                     "fail('hipMalloc'); gpu.quantize(c, INT4, w)"])
+def test_a_failed_call_leaves_no_error_for_the_next(run, failing):
+    run(f"""
+c = gpu.Context(0)
+cfg = Config(vocab=32, hidden=32, intermediate=32, layers=1, heads=2, kv_heads=2, head_dim=128)
+w = np.random.default_rng(0).standard_normal((32, 64)).astype(np.float32)
+try:
+    {failing}
+    assert False
+except gpu.FgError as e:
+    assert "failed" in str(e)
+got, want = gpu.quantize(c, INT4, w), host.quantize(INT4, w)
+assert np.array_equal(got.q, want.q) and np.array_equal(got.s, want.s)
 """)
