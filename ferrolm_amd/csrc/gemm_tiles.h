@@ -37,11 +37,11 @@ __device__ __forceinline__ uint32_t codes_bf16(uint32_t w, int b) {
 }
 
 // 1 KB per wave from global memory (base uniform, off the lane's byte) to LDS byte `lds` + 16 lane.
-// The compiler does not see the write: the kernel waits (vmcnt) and meets at a barrier itself. (M0
-// holds the LDS address; nothing else in these kernels uses it.)
+// The compiler does not see the write: the kernel waits (vmcnt) and meets at a barrier itself. M0
+// holds the LDS address.
 __device__ __forceinline__ void copy_to_lds(uint32_t lds, const uint8_t* base, uint32_t off) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
-                 : "memory");
+                 : "m0", "memory");
 }
 
 // The epilogues (internal.h) on one wave's 16 x 64 tile d (D layout), row tile rt, columns from

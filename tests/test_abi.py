@@ -91,3 +91,14 @@ def test_model_arrays_are_checked_before_upload():
         gpu.check_matrix(replace(good, s=np.zeros(64 * 2, np.float64)), "w")
     with pytest.raises(ValueError, match="bf16"):
         gpu.check_matrix(Matrix(0, 32, 32, bf16=np.zeros(32 * 32, np.float32)), "w")
+
+
+def test_inline_assembly_names_m0_where_it_writes_it():
+    """M0 is the compiler's too: an asm statement that sets it lists it among its clobbers."""
+    found = 0
+    for p in (ROOT / "ferrolm_amd" / "csrc").iterdir():
+        for stmt in re.findall(r"\basm\s+(?:volatile\s*)?\((.*?)\);", p.read_text(), flags=re.S):
+            if re.search(r"s_mov_b32 m0", stmt):
+                found += 1
+                assert '"m0"' in stmt.rsplit(":", 1)[1], (p, stmt)
+    assert found
