@@ -33,7 +33,7 @@ static std::set<Stream*> streams;
 static std::map<const void*, std::string> kernels;
 static std::map<std::string, int> failures;
 static thread_local int last_error;
-static int launched;
+static int launched, waits;
 
 using Lock = std::lock_guard<std::recursive_mutex>;
 
@@ -62,6 +62,7 @@ int fake_pending_default() {
     return (int)default_stream.queue.size();
 }
 int fake_launched() { return launched; }
+int fake_waits() { return waits; }
 
 void** __hipRegisterFatBinary(const void*) {
     static void* handle;
@@ -159,6 +160,7 @@ int hipStreamCreateWithFlags(void** s, unsigned) {
 }
 int hipStreamSynchronize(void* s) {
     Lock l(mu);
+    waits++;
     drain(of(s));
     return 0;
 }

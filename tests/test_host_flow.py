@@ -84,3 +84,40 @@ except gpu.FgError as e:
 got, want = gpu.quantize(c, INT4, w), host.quantize(INT4, w)
 assert np.array_equal(got.q, want.q) and np.array_equal(got.s, want.s)
 """)
+
+
+SHAPES = [(32, 32), (64, 2048), (1056, 1024), (2080, 2080), (160, 32800)]  # the last two over 16 MB, in panels and whole
+
+
+@pytest.mark.parametrize("refused", [None, ("hipHostMalloc", 1), ("hipStreamCreateWithFlags", 3),
+                                     ("hipEventCreateWithFlags", 8)])
+def test_quantizer_copies_with_and_without_staging(run, refused):
+    """Every size class of host copy, whole or in panels through staging slots, and with the slots refused:
+    codes and scales are the host quantizer's."""
+    run(f"""
+refused = {refused!r}
+rng = np.random.default_rng(0)
+for rows, cols in {SHAPES!r}:
+    w = rng.standard_normal((rows, cols)).astype(np.float32)
+    for imp in (None, rng.random(cols).astype(np.float32)):
+        c = gpu.Context(0)
+        if refused:
+            fail(*refused)
+        got, want = gpu.quantize(c, INT4, w, imp), host.quantize(INT4, w, imp)
+        assert np.array_equal(got.q, want.q) and np.array_equal(got.s, want.s), (rows, cols, imp is None)
+        if refused:
+            fail(refused[0], 0)
+        c.close()
+""")
+
+
+def test_a_small_quantizer_call_waits_once(run):
+    """Its copies are queued one after the other and waited for together."""
+    run("""
+c = gpu.Context(0)
+w = np.random.default_rng(0).standard_normal((64, 2048)).astype(np.float32)
+for imp in (None, np.ones(2048, np.float32)):
+    before = fake.fake_waits()
+    gpu.quantize(c, INT8, w, imp)
+    assert fake.fake_waits() == before + 1
+""")
