@@ -395,11 +395,17 @@ void launch_pack_bf16(hipStream_t st, const float* w, int rows, int K, uint32_t*
 
 void launch_mm_exact(hipStream_t st, int kind, const float* x, int m, int K, const uint32_t* wt, const float* s,
                      int rows, float* y) {
-    const dim3 grid((rows + 255) / 256, (m + kMmRows - 1) / kMmRows);
-    if (kind == BF16)
-        hipLaunchKernelGGL((k_mm_exact<true>), grid, dim3(256), 0, st, x, m, K, wt, s, rows, y);
-    else
-        hipLaunchKernelGGL((k_mm_exact<false>), grid, dim3(256), 0, st, x, m, K, wt, s, rows, y);
+    constexpr int kMost = 65535 * kMmRows;  // a grid's y is at most 65,535
+    for (int i = 0; i < m; i += kMost) {
+        const int mi = std::min(kMost, m - i);
+        const float* xi = x + (size_t)i * K;
+        float* yi = y + (size_t)i * rows;
+        const dim3 grid((rows + 255) / 256, (mi + kMmRows - 1) / kMmRows);
+        if (kind == BF16)
+            hipLaunchKernelGGL((k_mm_exact<true>), grid, dim3(256), 0, st, xi, mi, K, wt, s, rows, yi);
+        else
+            hipLaunchKernelGGL((k_mm_exact<false>), grid, dim3(256), 0, st, xi, mi, K, wt, s, rows, yi);
+    }
 }
 
 size_t sq_err_work(int count, int64_t n) { return (size_t)count * ((n + kErrChunk - 1) / kErrChunk) * 32; }

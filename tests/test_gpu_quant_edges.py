@@ -71,3 +71,13 @@ def test_search_copies_a_large_matrix(ctx):
     assert got[1:4] == tuple(want[1:4])
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[4].q, want[4].q)
     assert np.array_equal(got[4].s, want[4].s)
+
+
+def test_search_over_more_rows_than_one_grid(ctx):
+    """524,280 rows fill a launch's grid; the rest are a second one's."""
+    rng = np.random.default_rng(5)
+    w = (0.02 * rng.standard_normal((32, 32))).astype(np.float32)
+    cal = rng.standard_normal((524_280 + 13, 32)).astype(np.float32)
+    got, want = gpu.awq_search(ctx, INT8, w, cal), oracle.awq_search(INT8, w, cal)
+    assert got[1:4] == tuple(want[1:4])
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[4].q, want[4].q)

@@ -121,3 +121,12 @@ for imp in (None, np.ones(2048, np.float32)):
     gpu.quantize(c, INT8, w, imp)
     assert fake.fake_waits() == before + 1
 """)
+
+
+def test_the_search_takes_many_calibration_rows(run):
+    """600,000 rows: more than one grid's worth of row groups."""
+    run("""
+c = gpu.Context(0)
+gpu.awq_search(c, INT8, np.ones((32, 32), np.float32), np.ones((600_000, 32), np.float32))
+assert 0 < fake.fake_widest() <= 65535
+""")
