@@ -227,7 +227,7 @@ __global__ __launch_bounds__(64 * NWN * NWK, 2) void k_mm(const GemvArgs a) {
 #pragma unroll
     for (int t = 0; t < 4; t++) tl[t] = min((col0 >> 4) + t, ntl - 1);
     // the k-block pairs, in stages of NWK; in a last stage that is not full the shares past the end
-    // take the last pair again, with its scales (BF16: its weights) zero
+    // have nothing to add (their loads and copies take the last pair again)
     const int NP = KB >> 1, ns = (NP + NWK - 1) / NWK;
 
     // block q of the wave's share of stage s, into buffer s & 1
@@ -256,24 +256,18 @@ __global__ __launch_bounds__(64 * NWN * NWK, 2) void k_mm(const GemvArgs a) {
             } else if (KIND == INT8) {
                 r.w[t] = *((const u32x4*)a.W + (tile * (KB >> 1) + pr) * 64 + lane);
             } else {
-                const u32x4 z = {0, 0, 0, 0};
 #pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    const u32x4 v = *((const u32x4*)a.W + (tile * KB + 2 * pr + j) * 64 + lane);
-                    r.w[2 * t + j] = NWK == 1 || s * NWK + kw < NP ? v : z;
-                }
+                for (int j = 0; j < 2; j++)
+                    r.w[2 * t + j] = *((const u32x4*)a.W + (tile * KB + 2 * pr + j) * 64 + lane);
             }
         }
     };
     auto load_scales = [&](int s, Scales& sc) {
         const int pr = min(s * NWK + kw, NP - 1), c = pr >> 1, half = pr & 1;
-        const float on = NWK == 1 || s * NWK + kw < NP ? 1.0f : 0.0f;
         if (Q)
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
+            for (int t = 0; t < 4; t++)
                 sc.v[t] = *((const f32x2*)a.S + (((size_t)tl[t] * KC + c) * 16 + (lane & 15)) * 2 + half);
-                if (NWK > 1) sc.v[t] *= on;
-            }
     };
     // the operands of k-block j, [n-tile][word of two inputs]; word w (of 16) converted
     u32x4 B[2][4];
@@ -304,6 +298,8 @@ __global__ __launch_bounds__(64 * NWN * NWK, 2) void k_mm(const GemvArgs a) {
         // stage s has landed, here and in every wave, and every wave is done with the other buffer
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
+        // (a product with a zero scale would not be zero where it has overflowed)
+        if (NWK > 1 && s * NWK + kw >= NP) return;
         if (KIND == BF16) load_weights(s + 1, next);
         load_scales(s + 1, scn);
         const bf16x8* st = (const bf16x8*)(smem + (s & 1) * STAGE + kw * (4 * RT * 1024)) + lane;

@@ -54,6 +54,22 @@ def test_products_of_every_tile_shape(ctx, kind, n, k, m):
     assert np.all(np.abs(y - (x.astype(np.float64) @ deq.T + b)) <= 2e-5 * scale + 1e-6)
 
 
+@pytest.mark.parametrize("kind", [INT8, INT4], ids=["int8", "int4"])
+@pytest.mark.parametrize("n,k,m", SHAPES[-4:])
+def test_an_overflow_in_the_last_inputs_stays_an_infinity(ctx, kind, n, k, m):
+    """35 k-blocks make 18 pairs: with four shares of K the last stage has work for two only, and what the
+    others hold of the last pair must not reach the sum (a zero times an infinity)."""
+    rng = np.random.default_rng(n + k + m)
+    w = (0.1 * rng.standard_normal((n, k))).astype(np.float32)
+    sign = np.where(np.arange(n) % 3, 1.0, -1.0).astype(np.float32)
+    w[:, k - 5] = sign  # the largest of its group: the largest codes
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[m // 2, k - 5] = 3e38
+    y = gpu.Mat(ctx, oracle.quantize(kind, w)).matmul(x)
+    assert np.array_equal(y[m // 2], sign * np.float32(np.inf))
+    assert np.isfinite(np.delete(y, m // 2, axis=0)).all()
+
+
 def test_output_aligned_to_a_float(ctx):
     hip = Hip()
     rng = np.random.default_rng(1)
