@@ -84,7 +84,14 @@ struct Carver {
 struct Stage {
     static constexpr int kThreads = 4, kSlotsEach = 2, kSlots = kThreads * kSlotsEach;
     static constexpr size_t kSlotIn = (size_t)4 << 20, kSlotOut = (size_t)1280 << 10;
-    static constexpr size_t kCopyMin = (size_t)4 << 20, kPanelsMin = (size_t)16 << 20;
+    // The smallest copies that take the slots, with what a call costs without and with them, in us.
+    // Up, the only large copy of a call (quantize, int4): 4 MB 249, 286; 8 MB 398, 584; 16 MB 698, 886;
+    // 24 MB 1007, 1096; 32 MB 1443, 1391. Up beside others (the AWQ search): 8 MB 1762, 1956; 16 MB of
+    // calibration rows 8312, 6863; 20 MB of weights 5583, 4131. Back: 4 MB 818, 789; 6 MB in the search
+    // 6022, 5841; 8 MB 1808, 1904. Whole panels gain from 2 MB on (8 MB 398, 342; 16 MB 698, 545), but
+    // the slots cost a context's first call 1.8 ms and 84 MB, so panels wait for a matrix of 16 MB.
+    static constexpr size_t kUpAlone = (size_t)28 << 20, kUpBeside = (size_t)16 << 20, kBack = (size_t)4 << 20;
+    static constexpr size_t kPanels = (size_t)16 << 20;
     char *pin = nullptr, *dev = nullptr;
     hipStream_t streams[kThreads] = {};
     hipEvent_t ev[kSlots] = {};
@@ -1209,16 +1216,16 @@ static int staged(fg_ctx* c, size_t chunks, const I& issue, const F& finish) {
     return 0;
 }
 
-// A copy between pageable host memory and the device: a small one queued on the context's stream,
-// for the caller to wait for, a large one complete on return. The runtime's
+// A copy between pageable host memory and the device: one below `from` bytes queued on the context's
+// stream, for the caller to wait for, a larger one through the slots, complete on return. The runtime's
 // own copy of pageable memory ran at 28 GB/s and one thread's memcpy into pinned memory at 32,
 // pinned memory to the device at 56, so slots filled by several threads keep the link busy. A
 // thread gets about eight chunks: fewer leave the link idle at both ends (50 MB took 2.05 ms in
 // chunks of 4 MB; 0.5 less in chunks of 1.5), and below 512 KB a chunk's calls cost more than its
 // bytes. (A wait after each small copy made the quantizer's small calls 3% slower.)
-static int copy_host(fg_ctx* c, void* dst, const void* src, size_t bytes, bool to_device) {
+static int copy_host(fg_ctx* c, void* dst, const void* src, size_t bytes, bool to_device, size_t from) {
     const hipMemcpyKind kind = to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
-    if (bytes < Stage::kCopyMin || !stage_ready(c->stage)) {
+    if (bytes < from || !stage_ready(c->stage)) {
         HIPCHK(hipMemcpyAsync(dst, src, bytes, kind, c->stream));
         return 0;
     }
@@ -2124,7 +2131,7 @@ int fg_quantize(fg_ctx* ctx, int32_t kind, int32_t rows, int32_t cols, const flo
     auto apart = [&](const void* o, size_t bytes) {  // results come back while weights are still being read
         return (const char*)o + bytes <= (const char*)w || (const char*)w + n * 4 <= (const char*)o;
     };
-    const bool split = n * 4 >= Stage::kPanelsMin && panel * 4 <= Stage::kSlotIn && apart(q, qb) && apart(s, sn * 4) &&
+    const bool split = n * 4 >= Stage::kPanels && panel * 4 <= Stage::kSlotIn && apart(q, qb) && apart(s, sn * 4) &&
                        stage_ready(ctx->stage);
     float *dw, *di, *ds;
     uint8_t* dq;
@@ -2139,12 +2146,13 @@ int fg_quantize(fg_ctx* ctx, int32_t kind, int32_t rows, int32_t cols, const flo
     DevBuf buf;
     if ((rc = dev_alloc(buf, layout(nullptr)))) return rc;
     layout(buf.p);
-    if (importance && (rc = copy_host(ctx, di, importance, ib, true))) return rc;
+    if (importance && (rc = copy_host(ctx, di, importance, ib, true, Stage::kUpAlone))) return rc;
     if (!split) {
-        if ((rc = copy_host(ctx, dw, w, n * 4, true))) return rc;
+        if ((rc = copy_host(ctx, dw, w, n * 4, true, Stage::kUpAlone))) return rc;
         launch_quantize(st, kind, rows, cols, dw, nullptr, importance ? di : nullptr, dq, nullptr, ds);
         HIPCHK(hipGetLastError());
-        if ((rc = copy_host(ctx, q, dq, qb, false)) || (rc = copy_host(ctx, s, ds, sn * 4, false))) return rc;
+        if ((rc = copy_host(ctx, q, dq, qb, false, Stage::kBack)) || (rc = copy_host(ctx, s, ds, sn * 4, false, Stage::kBack)))
+            return rc;
         HIPCHK(hipStreamSynchronize(st));
         return 0;
     }
@@ -2240,11 +2248,13 @@ int fg_awq_search(fg_ctx* ctx, int32_t kind, int32_t rows, int32_t k, const floa
             });
         } catch (...) {
         }
-        if ((rc = copy_host(ctx, dw, w, rk * 4, true)) || (rc = copy_host(ctx, dx, cal, mk * 4, true))) return rc;
+        if ((rc = copy_host(ctx, dw, w, rk * 4, true, Stage::kUpBeside)) ||
+            (rc = copy_host(ctx, dx, cal, mk * 4, true, Stage::kUpBeside)))
+            return rc;
         if (beside.t.joinable()) beside.t.join();
         if (!done) statistics();
     }
-    if ((rc = copy_host(ctx, dsc, host.data(), host.size() * 4, true))) return rc;
+    if ((rc = copy_host(ctx, dsc, host.data(), host.size() * 4, true, Stage::kUpBeside))) return rc;
     // the reference output, with the unquantized weights as bf16 (Matrix::from_f32)
     launch_pack_bf16(st, dw, rows, k, wt);
     launch_mm_exact(st, BF16, dx, m, k, wt, nullptr, rows, dyref);
@@ -2272,7 +2282,8 @@ int fg_awq_search(fg_ctx* ctx, int32_t kind, int32_t rows, int32_t k, const floa
     const float* bs = dsc + (size_t)best_step * 2 * k;
     launch_quantize(st, kind, rows, k, dw, bs, bs + k, dq, nullptr, ds);
     HIPCHK(hipGetLastError());
-    if ((rc = copy_host(ctx, q, dq, qb, false)) || (rc = copy_host(ctx, s, ds, sn * 4, false))) return rc;
+    if ((rc = copy_host(ctx, q, dq, qb, false, Stage::kBack)) || (rc = copy_host(ctx, s, ds, sn * 4, false, Stage::kBack)))
+        return rc;
     HIPCHK(hipStreamSynchronize(st));
     std::memcpy(scales, scales_of(best_step), (size_t)k * 4);
     choice->alpha = (float)best_step / 10.0f;

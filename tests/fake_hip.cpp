@@ -33,7 +33,7 @@ static std::set<Stream*> streams;
 static std::map<const void*, std::string> kernels;
 static std::map<std::string, int> failures;
 static thread_local int last_error;
-static int launched, waits, widest;
+static int launched, waits, widest, pinned;
 
 using Lock = std::lock_guard<std::recursive_mutex>;
 
@@ -63,6 +63,7 @@ int fake_pending_default() {
 }
 int fake_launched() { return launched; }
 int fake_waits() { return waits; }
+int fake_pinned() { return pinned; }  // pinned allocations
 int fake_widest() { return widest; }  // the largest grid y of a launch
 
 void** __hipRegisterFatBinary(const void*) {
@@ -135,7 +136,10 @@ static int make(void** p, size_t n, const char* name) {
     return 0;
 }
 int hipMalloc(void** p, size_t n) { return make(p, n, "hipMalloc"); }
-int hipHostMalloc(void** p, size_t n, unsigned) { return make(p, n, "hipHostMalloc"); }
+int hipHostMalloc(void** p, size_t n, unsigned) {
+    pinned++;
+    return make(p, n, "hipHostMalloc");
+}
 int hipFree(void* p) {
     Lock l(mu);
     drain(&default_stream);

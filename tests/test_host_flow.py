@@ -86,7 +86,7 @@ assert np.array_equal(got.q, want.q) and np.array_equal(got.s, want.s)
 """)
 
 
-SHAPES = [(32, 32), (64, 2048), (1056, 1024), (2080, 2080), (160, 32800)]  # the last two over 16 MB, in panels and whole
+SHAPES = [(32, 32), (64, 2048), (1056, 1024), (2080, 2080), (224, 32800)]  # the last two over 16 MB, in panels and whole
 
 
 @pytest.mark.parametrize("refused", [None, ("hipHostMalloc", 1), ("hipStreamCreateWithFlags", 3),
@@ -129,4 +129,15 @@ def test_the_search_takes_many_calibration_rows(run):
 c = gpu.Context(0)
 gpu.awq_search(c, INT8, np.ones((32, 32), np.float32), np.ones((600_000, 32), np.float32))
 assert 0 < fake.fake_widest() <= 65535
+""")
+
+
+@pytest.mark.parametrize("rows,cols,staged", [(1024, 1024, 0), (2048, 2016, 0), (2048, 2048, 1), (192, 32800, 0)])
+def test_the_quantizer_takes_the_staging_slots_for_large_matrices_only(run, rows, cols, staged):
+    """In panels from 16 MB on; whole (a panel of more than 4 MB) from 28 MB on: below, the runtime's own copies
+    are faster."""
+    run(f"""
+c = gpu.Context(0)
+gpu.quantize(c, INT4, np.ones(({rows}, {cols}), np.float32))
+assert fake.fake_pinned() == {staged}
 """)
