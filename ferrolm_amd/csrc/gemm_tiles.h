@@ -211,15 +211,19 @@ __global__ __launch_bounds__(64 * NWN * NWK, 2) void k_mm(const GemvArgs a) {
     const int wn = wave % NWN, kw = wave / NWN;
     const int RTt = (a.p_total + 3) >> 2, groups = (RTt + RT - 1) / RT, cg = (a.N + BN - 1) / BN;
     // Workgroup i runs on XCD i % 8: an XCD takes whole column groups, its row groups one after the
-    // other, so a column group's weights are read from memory once and then from that XCD's L2.
+    // other, so a column group's weights are read from memory once and then from that XCD's L2. Where
+    // the column groups are not a multiple of eight it takes an eighth of the tiles in that order (bf16
+    // 3584 x 3584, 272 rows: 41.2 -> 28.8 us; taking them so everywhere made int8 49152 x 576 3% slower).
     int cgi, gi;
     if (cg % 8 == 0) {
         const int y = blockIdx.x / 8;
         cgi = (int)(blockIdx.x % 8) + 8 * (y / groups);
         gi = y % groups;
     } else {
-        cgi = blockIdx.x / groups;
-        gi = blockIdx.x % groups;
+        const int tiles = cg * groups, xcd = blockIdx.x % 8;
+        const int at = xcd * (tiles / 8) + min(xcd, tiles % 8) + (int)(blockIdx.x / 8);
+        cgi = at / groups;
+        gi = at % groups;
     }
     const int rt0 = gi * RT, col0 = cgi * BN + wn * 64, ntl = a.N >> 4, KB = a.KB, KC = KB >> 2;
     // n-tiles past the end re-read the last one (their results are discarded)
