@@ -2083,6 +2083,15 @@ int fg_matmul_device(fg_ctx* ctx, const fg_mat* w, const float* x_dev, int32_t m
     return 0;
 }
 
+int fg_mm_tile(int32_t kind, int32_t n, int32_t k, int32_t m, int32_t* row_tiles, int32_t* col_waves, int32_t* k_shares) {
+    if (!row_tiles || !col_waves || !k_shares || kind < BF16 || kind > INT4 || n <= 0 || k <= 0 || n % 32 || m <= 0)
+        return fail(FG_E_ARG, "bad argument");
+    const int tile = m > kGemvRows ? mm_tile(kind, n, round_up((k + 31) / 32, 4), m, (m + 3) / 4, kKpartFloats) : -1;
+    *row_tiles = *col_waves = *k_shares = 0;
+    if (tile >= 0) mm_tile_size(tile, row_tiles, col_waves, k_shares);
+    return 0;
+}
+
 int fg_matmul_device_noalloc(fg_ctx* ctx, const fg_mat* w, const float* x_dev, int32_t m, float* y_dev) {
     if (!ctx || !w || !x_dev || !y_dev || m <= 0) return fail(FG_E_ARG, "bad argument");
     if (!ctx->scratch) return fail(FG_E_DEVICE, "no scratch address on this device");

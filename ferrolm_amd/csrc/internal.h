@@ -180,8 +180,17 @@ struct GemvArgs {
 // so their interval is the kernel's own execution time.
 void launch_gemv(hipStream_t st, int epi, const DMat& w, const GemvArgs& a, hipEvent_t start = nullptr,
                  hipEvent_t stop = nullptr);
-// The tiled GEMM (gemm.hip) for MM inputs: 1, or 0 when the product is not its size and nothing
-// was launched.
+// A product's variant of k_gemm (kernels.hip): row tiles per workgroup, 64-column sets, row groups, and
+// the workgroups that share K.
+struct GemmShape {
+    int rtw, cs, groups, ks;
+};
+GemmShape gemm_shape(int n_tiles, int kb, int N, int m, int p_total, size_t kpart_cap);
+// The tiled GEMM (gemm.hip) for MM inputs: which of its tile shapes a product of m rows in p_total
+// passes takes (-1: none, it is k_gemm's), their sizes, and the launch (0 when it is k_gemm's and
+// nothing was launched).
+int mm_tile(int kind, int N, int KB, int m, int p_total, size_t kpart_cap);
+void mm_tile_size(int tile, int* row_tiles, int* col_waves, int* k_shares);
 int launch_mm(hipStream_t st, int epi, const DMat& w, const GemvArgs& a, hipEvent_t e0, hipEvent_t e1);
 // The output projection of a fused bf16 layer split by query head (k_o_heads):
 // a.apart / a.amrec the attention's span partials and merge records, a.anh,

@@ -1417,18 +1417,10 @@ __global__ __launch_bounds__(256) void k_gemm_finish(const GemvArgs a) {
 }
 
 template <int KIND, int RTW, int CS>
-static void gemm_rtw(hipStream_t st, int epi, const DMat& w, const GemvArgs& a0, int groups, hipEvent_t e0,
+static void gemm_rtw(hipStream_t st, int epi, const DMat& w, const GemvArgs& a0, int groups, int ks, hipEvent_t e0,
                      hipEvent_t e1) {
-    // Split K across workgroups when the tiles alone leave most CUs idle: up
-    // to 256 workgroups, at least one k-block pair per wave and split, and the
-    // partial tiles within the workspace's kpart buffer.
     GemvArgs a = a0;
-    const int cg = (w.n_tiles + 4 * CS - 1) / (4 * CS), cg64 = (w.n_tiles + 3) / 4, np = w.kb / 2;
-    int ks = 1;
-    if (a.kpart)
-        while (ks < 8 && cg * groups * ks * 2 <= 256 && np / (ks * 2) >= 8 &&
-               (size_t)ks * 2 * a.m * a.N <= a.kpart_cap)
-            ks *= 2;
+    const int cg = (w.n_tiles + 4 * CS - 1) / (4 * CS), cg64 = (w.n_tiles + 3) / 4;
     a.ks = ks;
     const dim3 grid(cg, groups, ks);
     // timed from the start of the main kernel to the end of the split's finish
@@ -1451,11 +1443,9 @@ static void gemm_rtw(hipStream_t st, int epi, const DMat& w, const GemvArgs& a0,
     }
 }
 
-template <int KIND>
-static void gemm_kind(hipStream_t st, int epi, const DMat& w, const GemvArgs& a, hipEvent_t e0, hipEvent_t e1) {
-    // the tiled GEMM (gemm.hip) takes the products whose tiles fill the chip; what is left:
-    if (launch_mm(st, epi, w, a, e0, e1)) return;
-    const int rt = (a.p_total + 3) / 4, groups = (rt + 4) / 5, rtw = (rt + groups - 1) / groups;
+GemmShape gemm_shape(int n_tiles, int kb, int N, int m, int p_total, size_t kpart_cap) {
+    const int rt = (p_total + 3) / 4, groups = (rt + 4) / 5, rtw = (rt + groups - 1) / groups;
+    GemmShape g = {std::max(2, rtw), 1, groups, 1};
     // 128-column tiles (CS 2) for steps of 256 rows or more when they still make
     // 512 workgroups (measured on the 1.7B int4 prefill of 1024 tokens: 14.45
     // against 15.3 ms; with fewer workgroups, the 135M draft's prefill and the
@@ -1469,23 +1459,37 @@ static void gemm_kind(hipStream_t st, int epi, const DMat& w, const GemvArgs& a,
     // 8644-8650 -> 8383-8386 us, cfg3 at 32 sequences 5682 -> 5485 us. At 40
     // rows (three-tile groups) they were slower: cfg3 at 8 sequences 2562 ->
     // 2690 us.
-    if (rt >= 5 && rt < 16 && rtw == 5 && w.n_tiles >= 1024) {
-        gemm_rtw<KIND, 5, 2>(st, epi, w, a, groups, e0, e1);
-        return;
-    }
-    if (rt >= 16 && w.n_tiles < 256)
-        gemm_rtw<KIND, 2, 1>(st, epi, w, a, (rt + 1) / 2, e0, e1);
+    if (rt >= 5 && rt < 16 && rtw == 5 && n_tiles >= 1024)
+        g.cs = 2;
+    else if (rt >= 16 && n_tiles < 256)
+        g.rtw = 2;
+    else if (rt >= 16 && (n_tiles + 7) / 8 * groups >= 512)
+        g.rtw = 5, g.cs = 2;
+    if (g.cs == 1) g.groups = g.rtw == 5 ? groups : (rt + g.rtw - 1) / g.rtw;
+    // Split K across workgroups when the tiles alone leave most CUs idle: up
+    // to 256 workgroups, at least one k-block pair per wave and split, and the
+    // partial tiles within the workspace's kpart buffer.
+    const int cg = (n_tiles + 4 * g.cs - 1) / (4 * g.cs), np = kb / 2;
+    while (g.ks < 8 && cg * g.groups * g.ks * 2 <= 256 && np / (g.ks * 2) >= 8 && (size_t)g.ks * 2 * m * N <= kpart_cap)
+        g.ks *= 2;
+    return g;
+}
+
+template <int KIND>
+static void gemm_kind(hipStream_t st, int epi, const DMat& w, const GemvArgs& a, hipEvent_t e0, hipEvent_t e1) {
+    // the tiled GEMM (gemm.hip) takes the products that it is faster for; what is left:
+    if (launch_mm(st, epi, w, a, e0, e1)) return;
+    const GemmShape g = gemm_shape(w.n_tiles, w.kb, a.N, a.m, a.p_total, a.kpart ? a.kpart_cap : 0);
+    if (g.cs == 2)
+        gemm_rtw<KIND, 5, 2>(st, epi, w, a, g.groups, g.ks, e0, e1);
+    else if (g.rtw == 2)
+        gemm_rtw<KIND, 2, 1>(st, epi, w, a, g.groups, g.ks, e0, e1);
+    else if (g.rtw == 3)
+        gemm_rtw<KIND, 3, 1>(st, epi, w, a, g.groups, g.ks, e0, e1);
+    else if (g.rtw == 4)
+        gemm_rtw<KIND, 4, 1>(st, epi, w, a, g.groups, g.ks, e0, e1);
     else
-    if (rt >= 16 && (w.n_tiles + 7) / 8 * groups >= 512)
-        gemm_rtw<KIND, 5, 2>(st, epi, w, a, groups, e0, e1);
-    else if (rtw <= 2)
-        gemm_rtw<KIND, 2, 1>(st, epi, w, a, (rt + 1) / 2, e0, e1);
-    else if (rtw == 3)
-        gemm_rtw<KIND, 3, 1>(st, epi, w, a, (rt + 2) / 3, e0, e1);
-    else if (rtw == 4)
-        gemm_rtw<KIND, 4, 1>(st, epi, w, a, (rt + 3) / 4, e0, e1);
-    else
-        gemm_rtw<KIND, 5, 1>(st, epi, w, a, groups, e0, e1);
+        gemm_rtw<KIND, 5, 1>(st, epi, w, a, g.groups, g.ks, e0, e1);
 }
 
 template <int KIND, int NT, int EPI>

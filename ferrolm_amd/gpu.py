@@ -133,6 +133,7 @@ EXPORTS = {
     "fg_matmul": (C.c_int, [C.c_void_p, C.c_void_p, f32p, C.c_int32, f32p, f32p]),
     "fg_matmul_device": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p]),
     "fg_matmul_device_noalloc": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p]),
+    "fg_mm_tile": (C.c_int, [C.c_int32, C.c_int32, C.c_int32, C.c_int32, i32p, i32p, i32p]),
     "fg_quantize": (C.c_int, [C.c_void_p, C.c_int32, C.c_int32, C.c_int32, f32p, f32p, u8p, f32p]),
     "fg_awq_search": (C.c_int, [C.c_void_p, C.c_int32, C.c_int32, C.c_int32, f32p, C.c_int32, f32p, f32p,
                                 C.POINTER(FgAwqChoice), u8p, f32p]),
@@ -563,6 +564,14 @@ class Mat:
     def __del__(self):
         if lib is not None:  # at interpreter exit the module's globals are already cleared
             self.close()
+
+
+def mm_tile(kind: int, n: int, k: int, m: int) -> tuple:
+    """The tile (row tiles of 16, waves of 64 columns, shares of K) that a product of m rows with an
+    n x k matrix takes, (0, 0, 0) where it is not the tiled GEMM's (fg_mm_tile; needs no device)."""
+    out = np.zeros(3, np.int32)
+    check(lib().fg_mm_tile(kind, n, k, m, *(ptr(out[i:], i32p) for i in range(3))))
+    return tuple(int(v) for v in out)
 
 
 def _qmatrix_buffers(kind: int, rows: int, cols: int):

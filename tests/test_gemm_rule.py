@@ -1,0 +1,46 @@
+"""Which kernel a product takes, without a device: the tiled GEMM where it was
+measured faster than the other one, by more than the measurement's noise, and
+not where it was slower (us of each beside the sizes)."""
+import pytest
+
+from ferrolm_amd import gpu
+from ferrolm_amd.weights import BF16, INT4, INT8
+
+
+# k_gemm's time, the tile's that the tile counts alone would choose
+@pytest.mark.parametrize("kind,n,k,m", [
+    (BF16, 4096, 4096, 256),    # 29.4, 34.5
+    (BF16, 4096, 4096, 320),    # 33.9, 39.8
+    (BF16, 2048, 2048, 400),    # 20.1, 23.0
+    (BF16, 2048, 2048, 1024),   # 32.6, 36.2
+    (BF16, 2048, 8192, 384),    # 51.3, 57.5
+    (BF16, 16384, 2048, 160),   # 32.2, 36.5
+    (BF16, 3584, 3584, 272),    # 27.4, 41.2
+    (BF16, 3072, 2048, 832),    # 36.0, 43.0
+    (INT4, 4096, 4096, 288),    # 38.2, 41.4
+    (INT4, 2048, 2048, 320),    # 20.9, 22.8
+    (INT4, 5120, 960, 224),     # 15.6, 18.8
+    (INT4, 7168, 2560, 160),    # 1.22 times
+    (INT4, 3072, 576, 832),     # 23.9, 27.1
+    (INT8, 5120, 960, 240),     # 15.7, 18.1
+    (INT8, 3072, 576, 512),     # 16.9, 18.5
+    (INT8, 4096, 1024, 256),    # 1.10 times
+])
+def test_products_that_are_slower_on_the_tiles_stay_off_them(kind, n, k, m):
+    assert gpu.mm_tile(kind, n, k, m) == (0, 0, 0)
+
+
+@pytest.mark.parametrize("kind,n,k,m", [
+    (INT4, 16384, 2048, 1024), (INT4, 6144, 2048, 1024), (INT4, 2048, 8192, 1024), (INT4, 28672, 4096, 80),
+    (INT8, 16384, 2048, 160), (INT8, 2048, 2048, 576), (INT8, 960, 2560, 777), (BF16, 49152, 576, 33),
+    (BF16, 6144, 2048, 512), (BF16, 2048, 8192, 1024), (INT8, 49152, 576, 33)])
+def test_products_that_gain_take_the_tiles(kind, n, k, m):
+    assert gpu.mm_tile(kind, n, k, m)[0]
+
+
+def test_small_products_are_not_the_tiles():
+    for kind in (BF16, INT8, INT4):
+        for m in (1, 15, 16, 32):
+            assert gpu.mm_tile(kind, 49152, 2048, m) == (0, 0, 0)
+    with pytest.raises(gpu.FgError, match="bad argument"):
+        gpu.mm_tile(INT4, 100, 2048, 64)

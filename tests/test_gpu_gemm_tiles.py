@@ -1,9 +1,9 @@
-"""The tiled GEMM at the edges of its tiles: one product for each tile shape,
-with outputs that are not a multiple of 64 or 128, rows that are not one of 16,
-an input of 5 k-blocks (padded to 8, so some shares of K have one stage and some
-none left) and one of 35 (padded to 36: a last stage that is not full); outputs
-into a buffer aligned to a float only; and a forward whose projections take it
-with every epilogue.
+"""The tiled GEMM at the edges of its tiles: products for each tile shape (which
+one a product takes is asserted), with outputs that are not a multiple of 64 or
+128, rows that are not one of 16, an input of 5 k-blocks (padded to 8, so some
+shares of K have one stage and some none left), of 35 (padded to 36: a last stage
+that is not full) and of 65; outputs into a buffer aligned to a float only; and
+forwards, one of them with every projection and so every epilogue on the tiles.
 
 A product's rows are held as two bf16 pieces (2^-17 of each input) and summed in
 f32, so |y - exact| <= 2e-5 * sum|x||w| as in the other products' tests."""
@@ -20,17 +20,16 @@ from test_zz_no_alloc import Hip
 
 pytestmark = pytest.mark.gpu
 
-# (outputs, inputs, rows): the shape's tile of row tiles x 64-column waves x K shares
-SHAPES = [(10016, 160, 1000),   # 8 x 4 x 1
-          (16448, 160, 400),    # 5 x 4 x 1
-          (9440, 160, 517),     # 8 x 4 x 2
-          (16448, 160, 200),    # 5 x 2 x 2
-          (16448, 160, 83),     # 4 x 2 x 2
-          (11456, 160, 129),    # 5 x 2 x 4
-          (6560, 160, 200),     # 4 x 2 x 4
-          (11456, 160, 67),     # 3 x 2 x 4
-          (1856, 1120, 300),    # 2 x 2 x 4
-          (16448, 1120, 200), (11456, 1120, 129), (6560, 1120, 200)]
+# (outputs, inputs, rows), and the tile that the product takes: row tiles, 64-column waves, K shares
+# (None: not the same one for every weight kind)
+SHAPES = [(10016, 160, 1000), (16448, 160, 400), (9440, 160, 517), (16448, 160, 200), (16448, 160, 83),
+          (11456, 160, 129), (6560, 160, 200), (11456, 160, 67), (1856, 1120, 300),
+          (16448, 1120, 200), (11456, 1120, 129), (6560, 1120, 200),
+          (16448, 160, 129), (8416, 160, 129), (1856, 2080, 300), (11456, 1120, 83), (9440, 1120, 517)]
+TILES = [(8, 4, 1), (5, 4, 1), (8, 4, 2), (5, 2, 2), None,
+         (5, 2, 4), (4, 2, 4), None, None,
+         (5, 2, 2), (5, 2, 4), (4, 2, 4),
+         (4, 2, 2), (3, 2, 4), (2, 2, 4), (3, 2, 4), (8, 4, 2)]
 
 
 def _matrix(kind, n, k, rng):
@@ -43,6 +42,8 @@ def _matrix(kind, n, k, rng):
 @pytest.mark.parametrize("kind", [BF16, INT8, INT4], ids=["bf16", "int8", "int4"])
 @pytest.mark.parametrize("n,k,m", SHAPES)
 def test_products_of_every_tile_shape(ctx, kind, n, k, m):
+    tile = TILES[SHAPES.index((n, k, m))]
+    assert tile is None or gpu.mm_tile(kind, n, k, m) == tile
     rng = np.random.default_rng(n + k + m)
     w = _matrix(kind, n, k, rng)
     x = rng.standard_normal((m, k)).astype(np.float32)
@@ -55,7 +56,7 @@ def test_products_of_every_tile_shape(ctx, kind, n, k, m):
 
 
 @pytest.mark.parametrize("kind", [INT8, INT4], ids=["int8", "int4"])
-@pytest.mark.parametrize("n,k,m", SHAPES[-4:])
+@pytest.mark.parametrize("n,k,m", [(1856, 1120, 300), (16448, 1120, 200), (11456, 1120, 129), (6560, 1120, 200)])
 def test_an_overflow_in_the_last_inputs_stays_an_infinity(ctx, kind, n, k, m):
     """35 k-blocks make 18 pairs: with four shares of K the last stage has work for two only, and what the
     others hold of the last pair must not reach the sum (a zero times an infinity)."""
@@ -91,16 +92,29 @@ def test_output_aligned_to_a_float(ctx):
     assert got[1][0] == 7.0 and np.all(got[1][m * n + 1:] == 7.0)
 
 
+# hidden, intermediate, heads of 32, kv heads, vocab, rows
+WIDE = (1056, 4256, 33, 11, 6560, 600)  # 33 and 133 k-blocks; the head's rows on one tile, the rest as the rule has it
+EVERY = (1440, 1440, 45, 15, 2080, 517)  # 45 k-blocks (padded to 48) everywhere, rows past a tile
+
+
+def test_every_projection_takes_the_tiles():
+    h, i, heads, kv, vocab, n = EVERY
+    for kind in (BF16, INT8, INT4):
+        for out, inp in (((heads + 2 * kv) * 32, h), (h, heads * 32), (2 * i, h), (h, i)):
+            assert gpu.mm_tile(kind, out, inp, n)[0], (kind, out, inp)
+    assert gpu.mm_tile(BF16, vocab, h, n)[0]
+
+
 @pytest.mark.parametrize("kind", [BF16, INT8, INT4], ids=["bf16", "int8", "int4"])
-def test_forward_on_the_tiles_matches_oracle(ctx, kind):
-    """600 rows of a 1056-wide model (33 k-blocks, padded to 36), two layers: q/k/v with a bias, o, gate/up,
-    down (two k-blocks of padding after its output) and the lm_head, logits, hidden states and cache slots
-    within 1e-4 of the oracle."""
+@pytest.mark.parametrize("dims", [WIDE, EVERY], ids=["wide", "every"])
+def test_forward_on_the_tiles_matches_oracle(ctx, kind, dims):
+    """Two layers: q/k/v with a bias, o, gate/up, down (its padding after the last output's k-block too) and the
+    lm_head, logits, hidden states and cache slots within 1e-4 of the oracle."""
     from ferrolm_amd.synth import quantize_model, random_model
-    cfg = Config(vocab=6560, hidden=1056, intermediate=4256, layers=2, heads=33, kv_heads=11, head_dim=32,
+    h, i, heads, kv_heads, vocab, n = dims
+    cfg = Config(vocab=vocab, hidden=h, intermediate=i, layers=2, heads=heads, kv_heads=kv_heads, head_dim=32,
                  rms_eps=1e-5, max_position=1024, qkv_bias=True)
     hm = quantize_model(random_model(cfg, seed=7, std=0.03), kind)
-    n = 600
     prompt = [int(t) for t in np.random.default_rng(8).integers(0, cfg.vocab, n)]
     blocks = (n + 15) // 16
     table = [(i * 7) % blocks for i in range(blocks)]
