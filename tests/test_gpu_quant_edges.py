@@ -81,3 +81,19 @@ def test_search_over_more_rows_than_one_grid(ctx):
     got, want = gpu.awq_search(ctx, INT8, w, cal), oracle.awq_search(INT8, w, cal)
     assert got[1:4] == tuple(want[1:4])
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[4].q, want[4].q)
+
+
+@pytest.mark.parametrize("row", [0, 300, 600])
+def test_search_errors_that_are_not_finite(ctx, row):
+    """A calibration row whose outputs overflow, in the first, a middle and the last chunk of 8192 error terms:
+    such a chunk has no map and its terms are added one by one. (The row's squares are still finite: the
+    importances, and so the codes, are ordinary.)"""
+    rng = np.random.default_rng(row)
+    w = (1e20 * rng.standard_normal((32, 160))).astype(np.float32)
+    cal = rng.standard_normal((601, 160)).astype(np.float32)
+    cal[row, 7:11] = 1e19
+    got, want = gpu.awq_search(ctx, INT8, w, cal), oracle.awq_search(INT8, w, cal)
+    assert not np.isfinite(want[2])
+    assert np.array_equal(np.float64(got[1:4]), np.float64(want[1:4]), equal_nan=True)
+    assert np.array_equal(got[0], want[0])
+    assert np.array_equal(got[4].s, want[4].s) and np.array_equal(got[4].q, want[4].q)
