@@ -551,8 +551,12 @@ static int build_plan(const fg_config& c, const fg_kv& kv, int max_pos, const Ch
     // 2806 -> 2768, 512 in 384 parts 5793 -> 5654, in 640 5509, 1024 rows 9947 -> 9404; 135M: 256 rows
     // (97 parts) 1719 -> 1680, 400 1939 -> 1849, 777 2790 -> 2340 in 423 parts, 2468 in 750; 8B (hd
     // 128): 64 rows (32 parts) 1380 -> 1423, 160 (144) 2142 -> 2175, 256 (320) 2883 -> 2862, 1024
-    // 8864 -> 8590. Batches with shorter chunks leave most of an item's 64 queries empty: from 256
-    // rows and parts on.
+    // 8864 -> 8590. A chunk that fills an item by one row more leaves the next item nearly empty, and
+    // is even or better all the same (verify batches of a six-layer model, us per forward: 16 sequences
+    // of 5 rows at position 1000, 16 heads a kv head, 819 -> 779, 32 of 5 1159 -> 1126; 8 heads, 16 of 9
+    // 1035 -> 1036, 32 of 9 1498 -> 1517; 16 of 4, which fill theirs, 723 -> 679; hd 128, 8 heads, 32 of 9
+    // 1521 -> 1517). Batches with shorter chunks leave most of an item's 64 queries empty: from 256 rows
+    // and parts on.
     const int rf = 2 * (attn_qmax(c.head_dim) / group);
     const int fblk = kFlashBlock(c.head_dim);
     int fpart = kFlashPart;
@@ -606,7 +610,7 @@ static int build_plan(const fg_config& c, const fg_kv& kv, int max_pos, const Ch
             const int boff = (int)P.btab.size();
             for (int b = 0; b < used; b++) P.btab.push_back((int32_t)k.blocks[b]);
             for (int r0 = 0; r0 < k.n; r0 += rf) {
-                // an item whose rows see more than kFlashBlocks blocks of 64 positions
+                // an item whose rows see more than fpart positions
                 // is split into parts of even length, each writing its own partials
                 // (the merge combines them as spans)
                 const int nr = std::min(rf, k.n - r0), L = k.pos + r0 + nr, nb = (L + fblk - 1) / fblk;

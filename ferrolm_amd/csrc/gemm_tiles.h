@@ -12,16 +12,18 @@
 // from LDS by NWN waves. The K shares' sums meet in LDS, each share finishing some of
 // the row tiles, and the epilogues run on a wave's own 16 x 64 tiles, without barriers.
 //
-// Bound: the issue of a SIMD's matrix and vector instructions. The group scale is
-// applied to every k-block's product (four FMAs for every two MFMAs) and a weight's
-// conversion takes about 1.7 operations; measured alone, an MFMA of 16 x 16 x 32 and
-// two FMAs take 20 cycles with two waves per SIMD, 16 without the FMAs. So a step's
-// MFMAs, FMAs, conversions and copies are interleaved by hand and two waves share each
-// SIMD. 1024 rows, int4: 16384 x 2048 226 -> 137 us (1000 TFLOP/s of bf16 MFMA
-// instructions; a large bf16 matrix product reaches 1380 on this card), 6144 x 2048
-// 93 -> 67, 2048 x 8192 125 -> 82, 28672 x 4096 685 -> 428; 80 rows of 28672 x 4096
-// 62 -> 50, 160 rows 120 -> 85 us. Three stages in LDS with one workgroup per CU were
-// no faster for single tiles and slower for full ones (16384 x 2048 158 us).
+// Bound: the issue of a SIMD's matrix and vector instructions, and on tiles of few rows what a stage
+// costs whatever its rows. The group scale is applied to every k-block's product (four FMAs for every
+// two MFMAs) and a weight's conversion takes about 1.7 operations; measured alone, an MFMA of 16 x 16 x
+// 32 and two FMAs take 20 cycles with two waves per SIMD, 16 without the FMAs. So a step's MFMAs, FMAs,
+// conversions and copies are interleaved by hand and two waves share each SIMD. A row tile of a stage is
+// then 0.21 us of MFMA issue, 0.27 with the FMAs; the four-share tiles take 0.35 us for each row tile and
+// 0.27 (bf16), 0.46 (int8) or 0.58 us (int4) besides (launch_mm's costs): a stage opens with a wait for
+// every load in flight and a barrier, and with two to five row tiles little is left to cover them.
+// Whole products of int4 weights, the packing of their inputs included, k_gemm -> here: 1024 rows, 16384
+// x 2048 217 -> 153 us, 6144 x 2048 95 -> 77, 2048 x 8192 134 -> 96, 28672 x 4096 677 -> 458; of 28672 x
+// 4096, 80 rows 60 -> 52, 160 rows 115 -> 92 us. Three stages in LDS with one workgroup per CU were no
+// faster for single tiles and slower for full ones (16384 x 2048 158 us for the product alone, 137 with two).
 #pragma once
 #include "devutil.h"
 

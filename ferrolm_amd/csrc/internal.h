@@ -266,8 +266,9 @@ constexpr int kAttnMfmaQueries = 16;
 // draft's 3 x 32 +12 us per step; the cfg2 verify's 32 x 32 unchanged).
 constexpr int kAttnDecWorkgroups = 1024;
 // Positions per block of the flash attention items, the most per part of an item, and the
-// workgroups below which a launch of full items takes shorter parts (one and a half a CU; more
-// parts than it takes to get there cost more in the merge than they gain).
+// workgroups below which a launch of full items takes shorter parts. The line lies between two
+// measured prompts of the 135M model: halved from 399 parts (1024 tokens) 2.81-2.94 ms against
+// 2.95-2.97 whole, from 423 (777 tokens) 2.47 against 2.34 (more parts cost more in the merge).
 constexpr int kFlashBlock(int hd) { return hd >= 128 ? 32 : 64; }
 constexpr int kFlashPart = 256;
 constexpr int kFlashParts = 400;

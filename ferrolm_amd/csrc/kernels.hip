@@ -1446,19 +1446,17 @@ static void gemm_rtw(hipStream_t st, int epi, const DMat& w, const GemvArgs& a0,
 GemmShape gemm_shape(int n_tiles, int kb, int N, int m, int p_total, size_t kpart_cap) {
     const int rt = (p_total + 3) / 4, groups = (rt + 4) / 5, rtw = (rt + groups - 1) / groups;
     GemmShape g = {std::max(2, rtw), 1, groups, 1};
-    // 128-column tiles (CS 2) for steps of 256 rows or more when they still make
-    // 512 workgroups (measured on the 1.7B int4 prefill of 1024 tokens: 14.45
-    // against 15.3 ms; with fewer workgroups, the 135M draft's prefill and the
-    // 160-row verify steps ran slower: 4.54 against 4.0 ms, 7.42 against 6.80 ms)
-    // Steps of 256 rows or more into fewer than 4096 outputs: row groups of two
-    // tiles, for more workgroups (measured on the cfg2 prompt's forwards: the
-    // 135M draft 3.97 -> 3.31 ms, the 1.7B target's o and down 14.13 -> 14.03 ms
-    // per forward)
-    // 80 to 160 rows into 16384 or more outputs (gate/up and the lm_heads of the
-    // batched verifies): 128-column tiles too. Same-box A/B: cfg4 verify
-    // 8644-8650 -> 8383-8386 us, cfg3 at 32 sequences 5682 -> 5485 us. At 40
-    // rows (three-tile groups) they were slower: cfg3 at 8 sequences 2562 ->
-    // 2690 us.
+    // What each rule is for among the products that the tiled GEMM leaves; the figures of forwards and
+    // steps were taken when all of their products ran here.
+    // Steps of 256 rows or more into fewer than 4096 outputs: row groups of two tiles, for more
+    // workgroups (the 135M draft's prompt of 1024 tokens 3.97 -> 3.31 ms; now its q/k/v and o, and
+    // bf16 products of 2048 inputs or fewer: 3072 x 2048 at 512 rows 25.5 us, 29.4 on the tiles).
+    // 128-column tiles (CS 2): for 80 to 160 rows into 16384 or more outputs (cfg4 verify 8644-8650 ->
+    // 8383-8386 us; now bf16 only: 16384 x 2048 at 160 rows 32.5 us, 36.2 on the tiles, 28672 x 4096 at
+    // 80 rows 50.9, 57.9; at 40 rows, three-tile groups, they were slower: cfg3 at 8 sequences 2562 ->
+    // 2690 us), and for 256 rows or more where they make 512 workgroups (the 1.7B int4 prompt of 1024
+    // tokens 14.45 against 15.3 ms; now what launch_mm's first choice of shape has too few tiles for:
+    // 6144 outputs at 801 to 896 rows, 5120 x 5120 at 1024).
     if (rt >= 5 && rt < 16 && rtw == 5 && n_tiles >= 1024)
         g.cs = 2;
     else if (rt >= 16 && n_tiles < 256)
