@@ -124,11 +124,17 @@ int mm_tile(int kind, int N, int KB, int m, int p_total, size_t kpart_cap) {
     // 23.5 against 18.8).
     if (rt < 5) return tile;
     const GemmShape g = gemm_shape(N / 16, KB, N, m, p_total, kpart_cap);
+    const int cg = (N / 16 + 4 * g.cs - 1) / (4 * g.cs), wgs = cg * g.groups;
+    // Past 1024 rows (211 products up to 32768, each on both) activations no longer stay in the L2s, which
+    // the model does not know, and the tiles win, but for bf16 on k_gemm's two-row tiles up to 4096 rows
+    // (960 x 576 at 2048: 22.2 against 26.4 us; at 16384 114.5 against 94.7). Seven of the bf16 products
+    // are over 3% slower on the tiles, up to 1.10 times, none of int8 and four of int4, up to 1.07.
+    if (rt > 64)
+        return kind == BF16 && g.rtw == 2 && m <= 4096 && (KB <= 32 || (KB <= 64 && cg % 8 == 0)) ? -1 : tile;
     // Where k_gemm does better than its model: its two-row tiles, three workgroups on a CU, on short K
     // (3072 x 576 at 832 rows, int4: 23.9 against 27.1), for bf16 up to 2048 inputs when an XCD keeps its
     // column groups (3072 x 2048 at 832 rows: 36.0 against 43.0); and for bf16 one full round of its
     // largest tiles without a split (16384 x 2048 at 160 rows: 32.8 against 36.6).
-    const int cg = (N / 16 + 4 * g.cs - 1) / (4 * g.cs), wgs = cg * g.groups;
     if (g.rtw == 2 && (KB < 32 || (kind == BF16 && KB <= 64 && cg % 8 == 0))) return -1;
     if (kind == BF16 && g.rtw >= 4 && g.ks == 1 && wgs > 192 && wgs <= 256) return -1;
     const Costs& c = kCosts[kind == BF16 ? 0 : kind == INT8 ? 1 : 2];

@@ -25,6 +25,8 @@ from ferrolm_amd.weights import BF16, INT4, INT8
     (INT8, 5120, 960, 240),     # 15.7, 18.1
     (INT8, 3072, 576, 512),     # 16.9, 18.5
     (INT8, 4096, 1024, 256),    # 1.10 times
+    (BF16, 960, 576, 2048),     # 22.2, 26.4
+    (BF16, 960, 960, 2048),     # 28.1, 32.0
 ])
 def test_products_that_are_slower_on_the_tiles_stay_off_them(kind, n, k, m):
     assert gpu.mm_tile(kind, n, k, m) == (0, 0, 0)
@@ -33,7 +35,10 @@ def test_products_that_are_slower_on_the_tiles_stay_off_them(kind, n, k, m):
 @pytest.mark.parametrize("kind,n,k,m", [
     (INT4, 16384, 2048, 1024), (INT4, 6144, 2048, 1024), (INT4, 2048, 8192, 1024), (INT4, 28672, 4096, 80),
     (INT8, 16384, 2048, 160), (INT8, 2048, 2048, 576), (INT8, 960, 2560, 777), (BF16, 49152, 576, 33),
-    (BF16, 6144, 2048, 512), (BF16, 2048, 8192, 1024), (INT8, 49152, 576, 33)])
+    (BF16, 6144, 2048, 512), (BF16, 2048, 8192, 1024), (INT8, 49152, 576, 33),
+    # 572.9 to 419.7, 172.1 to 105.8, 863.1 to 657.7, 681.2 to 450.8, 307.2 to 204.6
+    (BF16, 3072, 576, 32768), (BF16, 960, 2560, 6144), (BF16, 2048, 2048, 32768), (INT8, 3072, 576, 32768),
+    (INT4, 960, 576, 32768)])
 def test_products_that_gain_take_the_tiles(kind, n, k, m):
     assert gpu.mm_tile(kind, n, k, m)[0]
 
