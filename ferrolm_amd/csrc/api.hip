@@ -2087,10 +2087,14 @@ int fg_matmul_device(fg_ctx* ctx, const fg_mat* w, const float* x_dev, int32_t m
     return 0;
 }
 
-int fg_mm_tile(int32_t kind, int32_t n, int32_t k, int32_t m, int32_t* row_tiles, int32_t* col_waves, int32_t* k_shares) {
-    if (!row_tiles || !col_waves || !k_shares || kind < BF16 || kind > INT4 || n <= 0 || k <= 0 || n % 32 || m <= 0)
+int fg_mm_tile(int32_t use, int32_t kind, int32_t n, int32_t k, int32_t m, int32_t* row_tiles, int32_t* col_waves,
+               int32_t* k_shares) {
+    static const int epi[] = {EPI_STORE, EPI_QKV, EPI_RESID, EPI_SILU, EPI_ARGMAX};
+    if (!row_tiles || !col_waves || !k_shares || use < 0 || use > 4 || kind < BF16 || kind > INT4 || n <= 0 ||
+        k <= 0 || n % 32 || m <= 0)
         return fail(FG_E_ARG, "bad argument");
-    const int tile = m > kGemvRows ? mm_tile(kind, n, round_up((k + 31) / 32, 4), m, (m + 3) / 4, kKpartFloats) : -1;
+    const int tile =
+        m > kGemvRows ? mm_tile(epi[use], kind, n, round_up((k + 31) / 32, 4), m, (m + 3) / 4, kKpartFloats) : -1;
     *row_tiles = *col_waves = *k_shares = 0;
     if (tile >= 0) mm_tile_size(tile, row_tiles, col_waves, k_shares);
     return 0;

@@ -25,13 +25,13 @@ static const struct {
     {5, 2, 4, 3.1f, 0.0f},  {4, 2, 4, 2.65f, 0.0f}, {3, 2, 4, 2.25f, 0.0f}, {2, 2, 4, 1.85f, 0.0f},
 };
 
-// What a product costs on the tiles and on k_gemm, in us, beyond what both pay (the packing of its
+// What a lone product costs on the tiles and on k_gemm, in us, beyond what both pay (the packing of its
 // inputs, the launches): per weight kind, a stage of each tile shape (kTiles' order) for a CU's only
 // workgroup and for two of four waves, and k_gemm's time for a k-block pair of each wave by row tiles
 // (2: one, two and three workgroups on a CU, 3: one and two, 4, 5, and 5 of 128 columns). A least
 // squares fit to 3500 products of 33 to 1024 rows, each run on k_gemm and on all nine shapes (37 sizes,
 // 576 to 49152 outputs, 576 to 14336 inputs); predicted over measured was 0.93 to 1.08 for nine in ten
-// on the tiles and 0.88 to 1.12 on k_gemm. With the rule below none of them is over 3% slower than on
+// on the tiles and 0.88 to 1.12 on k_gemm. With store_on_gemm none of them is over 3% slower than on
 // k_gemm; by tile counts alone 138 were, up to 1.22 times (bf16 4096 x 4096 at 320 rows: 33.9 against
 // 39.8 us, int4 5120 x 960 at 224: 15.6 against 18.8).
 struct Costs {
@@ -101,7 +101,51 @@ void mm_tile_size(int tile, int* row_tiles, int* col_waves, int* k_shares) {
     *k_shares = kTiles[tile].nwk;
 }
 
-int mm_tile(int kind, int N, int KB, int m, int p_total, size_t kpart_cap) {
+// Whether k_gemm is the faster for a forward's product with its epilogue: 3171 products of two-layer
+// models (33 to 4096 rows, eleven models of 576 to 4096 wide, all kinds), each on k_gemm and on the tiles.
+// q/k/v and gate/up (1629 of them) gain wherever the tiles are enough: 0.84, 0.80 and 0.82 of k_gemm's time
+// in the mean for q/k/v (bf16, int8, int4), 0.69, 0.69 and 0.71 for gate/up, none over 4% slower. Of o and
+// down, 47 were over 5% slower, up to 1.33 times; what they are is below, and with it one is, by 5.2%.
+static bool resid_on_gemm(int kind, int tile, int n, const GemmShape& g, int N) {
+    // k_gemm's tiles of four or five row tiles, one full round of the chip without a split (4096 x 14336 at 256
+    // to 320 rows: 1.28 to 1.33 times as long on the tiles in bf16, 1.17 to 1.25 in int4, 1.11 in int8)
+    const int wgs = (N + 64 * g.cs - 1) / (64 * g.cs) * g.groups;
+    if (g.rtw >= 4 && g.ks == 1 && wgs > 192 && wgs <= 256) return true;
+    if (kind != BF16) return false;
+    // bf16, whose weights take twice the loads and no conversion to hide them: two-row tiles (2048 x 8192 at
+    // 320 to 512 rows 1.25 to 1.31 times, 1536 wide even, narrower ones down to 0.71), three-row tiles in
+    // more than one round (2560 x 6912 at 1024 rows 1.25, 3072 x 8192 at 832 1.22, 4096 x 14336 at 704
+    // even), and four waves just past a round (2560 x 2560 at 1024 rows 1.08)
+    const auto& c = kTiles[tile];
+    if (c.rt == 2) return N >= 1536;
+    if (c.rt == 3) return n > 256;
+    return c.nwn * c.nwk == 4 && n > 256 && n <= 320;
+}
+
+// Whether k_gemm is the faster for a lone product.
+static bool store_on_gemm(int kind, int tile, int n, const GemmShape& g, int N, int KB, int m, int rt) {
+    const int cg = (N + 64 * g.cs - 1) / (64 * g.cs), wgs = cg * g.groups;
+    // Up to 64 rows only the widest products come here, and all of them gain (49152 x 576 at 33 rows, int8:
+    // 23.5 against 18.8 us).
+    if (rt < 5) return false;
+    // Past 1024 rows (211 products up to 32768, each on both) activations no longer stay in the L2s, which
+    // the model does not know, and the tiles win, but for bf16 on k_gemm's two-row tiles up to 4096 rows
+    // (960 x 576 at 2048: 22.2 against 26.4 us; at 16384 114.5 against 94.7). Seven of the bf16 products
+    // are over 3% slower on the tiles, up to 1.10 times, none of int8 and four of int4, up to 1.07.
+    if (rt > 64) return kind == BF16 && g.rtw == 2 && m <= 4096 && (KB <= 32 || (KB <= 64 && cg % 8 == 0));
+    // Where k_gemm does better than its model: its two-row tiles, three workgroups on a CU, on short K
+    // (3072 x 576 at 832 rows, int4: 23.9 against 27.1), for bf16 up to 2048 inputs when an XCD keeps its
+    // column groups (3072 x 2048 at 832 rows: 36.0 against 43.0); and for bf16 one full round of its
+    // largest tiles without a split (16384 x 2048 at 160 rows: 32.8 against 36.6).
+    if (g.rtw == 2 && (KB < 32 || (kind == BF16 && KB <= 64 && cg % 8 == 0))) return true;
+    if (kind == BF16 && g.rtw >= 4 && g.ks == 1 && wgs > 192 && wgs <= 256) return true;
+    const Costs& c = kCosts[kind == BF16 ? 0 : kind == INT8 ? 1 : 2];
+    const float tiles = tile_time(tile, n, tile_stages(tile, KB), c.one[tile], c.two[tile], c.round) +
+                        c.out * (float)m * (float)N * 1e-6f;
+    return tiles >= c.gain * gemm_time(c, g, kind, N, KB, m);
+}
+
+int mm_tile(int epi, int kind, int N, int KB, int m, int p_total, size_t kpart_cap) {
     const int rt = (p_total + 3) / 4;
     if (rt < 3) return -1;
     int tile = -1;
@@ -120,31 +164,15 @@ int mm_tile(int kind, int N, int KB, int m, int p_total, size_t kpart_cap) {
     // short K with two row tiles 960 x 576 at 1024 rows 14.5 against 16.2.
     const int n = tile_count(tile, N, rt);
     if (kTiles[tile].rt == 2 ? n < 150 || m < 256 || KB < 32 : n < 180) return -1;
-    // Up to 64 rows only the widest products come here, and all of them gain (49152 x 576 at 33 rows, int8:
-    // 23.5 against 18.8).
-    if (rt < 5) return tile;
+    if (epi != EPI_RESID && epi != EPI_STORE) return tile;
     const GemmShape g = gemm_shape(N / 16, KB, N, m, p_total, kpart_cap);
-    const int cg = (N / 16 + 4 * g.cs - 1) / (4 * g.cs), wgs = cg * g.groups;
-    // Past 1024 rows (211 products up to 32768, each on both) activations no longer stay in the L2s, which
-    // the model does not know, and the tiles win, but for bf16 on k_gemm's two-row tiles up to 4096 rows
-    // (960 x 576 at 2048: 22.2 against 26.4 us; at 16384 114.5 against 94.7). Seven of the bf16 products
-    // are over 3% slower on the tiles, up to 1.10 times, none of int8 and four of int4, up to 1.07.
-    if (rt > 64)
-        return kind == BF16 && g.rtw == 2 && m <= 4096 && (KB <= 32 || (KB <= 64 && cg % 8 == 0)) ? -1 : tile;
-    // Where k_gemm does better than its model: its two-row tiles, three workgroups on a CU, on short K
-    // (3072 x 576 at 832 rows, int4: 23.9 against 27.1), for bf16 up to 2048 inputs when an XCD keeps its
-    // column groups (3072 x 2048 at 832 rows: 36.0 against 43.0); and for bf16 one full round of its
-    // largest tiles without a split (16384 x 2048 at 160 rows: 32.8 against 36.6).
-    if (g.rtw == 2 && (KB < 32 || (kind == BF16 && KB <= 64 && cg % 8 == 0))) return -1;
-    if (kind == BF16 && g.rtw >= 4 && g.ks == 1 && wgs > 192 && wgs <= 256) return -1;
-    const Costs& c = kCosts[kind == BF16 ? 0 : kind == INT8 ? 1 : 2];
-    const float tiles = tile_time(tile, n, tile_stages(tile, KB), c.one[tile], c.two[tile], c.round) +
-                        c.out * (float)m * (float)N * 1e-6f;
-    return tiles < c.gain * gemm_time(c, g, kind, N, KB, m) ? tile : -1;
+    const bool other = epi == EPI_RESID ? resid_on_gemm(kind, tile, n, g, N)
+                                        : store_on_gemm(kind, tile, n, g, N, KB, m, rt);
+    return other ? -1 : tile;
 }
 
 int launch_mm(hipStream_t st, int epi, const DMat& w, const GemvArgs& a, hipEvent_t e0, hipEvent_t e1) {
-    const int tile = mm_tile(w.kind, a.N, a.KB, a.m, a.p_total, a.kpart ? a.kpart_cap : 0);
+    const int tile = mm_tile(epi, w.kind, a.N, a.KB, a.m, a.p_total, a.kpart ? a.kpart_cap : 0);
     if (tile < 0) return 0;
     if (w.kind == INT4)
         run_mm<INT4>(st, epi, tile, a, e0, e1);

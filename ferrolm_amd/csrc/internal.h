@@ -187,9 +187,9 @@ struct GemmShape {
 };
 GemmShape gemm_shape(int n_tiles, int kb, int N, int m, int p_total, size_t kpart_cap);
 // The tiled GEMM (gemm.hip) for MM inputs: which of its tile shapes a product of m rows in p_total
-// passes takes (-1: none, it is k_gemm's), their sizes, and the launch (0 when it is k_gemm's and
-// nothing was launched).
-int mm_tile(int kind, int N, int KB, int m, int p_total, size_t kpart_cap);
+// passes takes with an epilogue (-1: none, it is k_gemm's), their sizes, and the launch (0 when it is
+// k_gemm's and nothing was launched).
+int mm_tile(int epi, int kind, int N, int KB, int m, int p_total, size_t kpart_cap);
 void mm_tile_size(int tile, int* row_tiles, int* col_waves, int* k_shares);
 int launch_mm(hipStream_t st, int epi, const DMat& w, const GemvArgs& a, hipEvent_t e0, hipEvent_t e1);
 // The output projection of a fused bf16 layer split by query head (k_o_heads):

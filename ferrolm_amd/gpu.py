@@ -133,7 +133,7 @@ EXPORTS = {
     "fg_matmul": (C.c_int, [C.c_void_p, C.c_void_p, f32p, C.c_int32, f32p, f32p]),
     "fg_matmul_device": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p]),
     "fg_matmul_device_noalloc": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p]),
-    "fg_mm_tile": (C.c_int, [C.c_int32, C.c_int32, C.c_int32, C.c_int32, i32p, i32p, i32p]),
+    "fg_mm_tile": (C.c_int, [C.c_int32] * 5 + [i32p] * 3),
     "fg_quantize": (C.c_int, [C.c_void_p, C.c_int32, C.c_int32, C.c_int32, f32p, f32p, u8p, f32p]),
     "fg_awq_search": (C.c_int, [C.c_void_p, C.c_int32, C.c_int32, C.c_int32, f32p, C.c_int32, f32p, f32p,
                                 C.POINTER(FgAwqChoice), u8p, f32p]),
@@ -566,11 +566,13 @@ class Mat:
             self.close()
 
 
-def mm_tile(kind: int, n: int, k: int, m: int) -> tuple:
+def mm_tile(kind: int, n: int, k: int, m: int, use: str = "alone") -> tuple:
     """The tile (row tiles of 16, waves of 64 columns, shares of K) that a product of m rows with an
-    n x k matrix takes, (0, 0, 0) where it is not the tiled GEMM's (fg_mm_tile; needs no device)."""
+    n x k matrix takes, (0, 0, 0) where it is not the tiled GEMM's (fg_mm_tile; needs no device).
+    use: "alone", or in a forward "qkv", "resid" (o, down), "gate_up" or "head"."""
     out = np.zeros(3, np.int32)
-    check(lib().fg_mm_tile(kind, n, k, m, *(ptr(out[i:], i32p) for i in range(3))))
+    check(lib().fg_mm_tile(("alone", "qkv", "resid", "gate_up", "head").index(use), kind, n, k, m,
+                           *(ptr(out[i:], i32p) for i in range(3))))
     return tuple(int(v) for v in out)
 
 

@@ -304,9 +304,11 @@ int fg_matmul_device(fg_ctx* ctx, const fg_mat* w, const float* x_dev,
                      int32_t m, float* y_dev);
 /* Which tile of the tiled GEMM a product of m rows takes with a matrix of
  * this format (FG_BF16 ...), n outputs and k inputs: row tiles of 16, waves
- * of 64 columns, shares of K; all 0 where another kernel takes it. The rule
- * itself, for tests and measurements; needs no device. */
-int fg_mm_tile(int32_t kind, int32_t n, int32_t k, int32_t m,
+ * of 64 columns, shares of K; all 0 where another kernel takes it. use: 0 a
+ * product alone (fg_matmul), in a forward 1 q/k/v, 2 o or down, 3 gate/up,
+ * 4 the lm_head. The rule itself, for tests and measurements; needs no
+ * device. */
+int fg_mm_tile(int32_t use, int32_t kind, int32_t n, int32_t k, int32_t m,
                int32_t* row_tiles, int32_t* col_waves, int32_t* k_shares);
 /* fg_matmul_device without allocating: no counterpart in the reference; for
  * callers that cannot allocate device memory (HIP graph capture, tight

@@ -1,6 +1,6 @@
-"""Which kernel a product takes, without a device: the tiled GEMM where it was
-measured faster than the other one, by more than the measurement's noise, and
-not where it was slower (us of each beside the sizes)."""
+"""Which kernel a product takes, alone and as a forward's projection, without a
+device: the tiled GEMM where it was measured faster than the other one, and not
+where it was slower (the measurements stand beside the sizes)."""
 import pytest
 
 from ferrolm_amd import gpu
@@ -41,6 +41,37 @@ def test_products_that_are_slower_on_the_tiles_stay_off_them(kind, n, k, m):
     (INT4, 960, 576, 32768)])
 def test_products_that_gain_take_the_tiles(kind, n, k, m):
     assert gpu.mm_tile(kind, n, k, m)[0]
+
+
+# o and down of a forward, their time on the tile over k_gemm's
+@pytest.mark.parametrize("kind,n,k,m", [
+    (BF16, 2048, 8192, 320),    # 1.31
+    (BF16, 2048, 2048, 512),    # 1.10
+    (BF16, 4096, 14336, 256),   # 1.33
+    (BF16, 3072, 8192, 832),    # 1.22
+    (BF16, 2560, 6912, 1024),   # 1.25
+    (BF16, 2560, 2560, 1024),   # 1.08
+    (INT8, 4096, 14336, 320),   # 1.11
+    (INT4, 4096, 14336, 256),   # 1.25
+    (INT4, 4096, 4096, 272),    # 1.06
+])
+def test_residual_products_that_are_slower_on_the_tiles_stay_off_them(kind, n, k, m):
+    assert gpu.mm_tile(kind, n, k, m, "resid") == (0, 0, 0)
+
+
+# a forward's products that gain, though some of them would not alone; the ratio again
+@pytest.mark.parametrize("use,kind,n,k,m", [
+    ("gate_up", BF16, 3072, 576, 1024),    # 17.4 us, 22.5 on k_gemm
+    ("qkv", BF16, 3072, 2048, 832), ("resid", BF16, 576, 1536, 1024),  # 0.74
+    ("resid", BF16, 960, 2560, 1024),      # 0.73
+    ("resid", BF16, 2048, 8192, 1024),     # 0.89
+    ("resid", INT4, 2048, 8192, 320),      # 0.83
+    ("resid", INT8, 2048, 2048, 320),      # 0.84
+    ("resid", INT4, 4096, 14336, 384),     # 0.65
+    ("gate_up", INT4, 28672, 4096, 80), ("gate_up", INT8, 16384, 2048, 160), ("head", BF16, 128256, 4096, 80),
+    ("qkv", INT4, 6144, 2048, 1024)])
+def test_products_of_forwards_that_gain_take_the_tiles(use, kind, n, k, m):
+    assert gpu.mm_tile(kind, n, k, m, use)[0]
 
 
 def test_small_products_are_not_the_tiles():

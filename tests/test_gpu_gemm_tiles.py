@@ -100,9 +100,10 @@ EVERY = (1440, 1440, 45, 15, 2080, 517)  # 45 k-blocks (padded to 48) everywhere
 def test_every_projection_takes_the_tiles():
     h, i, heads, kv, vocab, n = EVERY
     for kind in (BF16, INT8, INT4):
-        for out, inp in (((heads + 2 * kv) * 32, h), (h, heads * 32), (2 * i, h), (h, i)):
-            assert gpu.mm_tile(kind, out, inp, n)[0], (kind, out, inp)
-    assert gpu.mm_tile(BF16, vocab, h, n)[0]
+        for use, out, inp in (("qkv", (heads + 2 * kv) * 32, h), ("resid", h, heads * 32), ("gate_up", 2 * i, h),
+                              ("resid", h, i)):
+            assert gpu.mm_tile(kind, out, inp, n, use)[0], (kind, use, out, inp)
+    assert gpu.mm_tile(BF16, vocab, h, n, "head")[0]
 
 
 @pytest.mark.parametrize("kind", [BF16, INT8, INT4], ids=["bf16", "int8", "int4"])
