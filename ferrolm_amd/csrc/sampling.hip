@@ -348,7 +348,7 @@ __global__ void k_accept_sampled(int n_seqs, int k, const SampleParams* __restri
 // Bound: the latency of eight dependent launches. 49,152 tokens, 4 rows: 2664
 // us for the whole distribution on one workgroup a row (its tiles of the sort
 // one after the other, its sums one lane each), 8008 us for the acceptance;
-// now 145 us (sort 4 x 14, sums 71) and 191 us.
+// now 140 us (sort 4 x 14, sums 71) and 200 us.
 // ---------------------------------------------------------------------------
 constexpr int kWideTile = 1024;  // tokens per workgroup
 
