@@ -1452,9 +1452,10 @@ GemmShape gemm_shape(int n_tiles, int kb, int N, int m, int p_total, size_t kpar
     // workgroups (the 135M draft's prompt of 1024 tokens 3.97 -> 3.31 ms; now its q/k/v and o, and
     // bf16 products of 2048 inputs or fewer: 3072 x 2048 at 512 rows 25.5 us, 29.4 on the tiles).
     // 128-column tiles (CS 2): for 80 to 160 rows into 16384 or more outputs (cfg4 verify 8644-8650 ->
-    // 8383-8386 us; now bf16 only: 16384 x 2048 at 160 rows 32.5 us, 36.2 on the tiles, 28672 x 4096 at
-    // 80 rows 50.9, 57.9; at 40 rows, three-tile groups, they were slower: cfg3 at 8 sequences 2562 ->
-    // 2690 us), and for 256 rows or more where they make 512 workgroups (the 1.7B int4 prompt of 1024
+    // 8383-8386 us; now lone bf16 products, 16384 x 2048 at 160 rows 32.5 us, 36.2 on the tiles, 28672 x
+    // 4096 at 80 rows 50.9, 57.9, and widths of any kind whose best shape makes too few tiles, 16640 to
+    // 22784 outputs at 80 rows; at 40 rows, three-tile groups, they were slower: cfg3 at 8 sequences
+    // 2562 -> 2690 us), and for 256 rows or more where they make 512 workgroups (the 1.7B int4 prompt of 1024
     // tokens 14.45 against 15.3 ms; now what launch_mm's first choice of shape has too few tiles for:
     // 6144 outputs at 801 to 896 rows, 5120 x 5120 at 1024).
     if (rt >= 5 && rt < 16 && rtw == 5 && n_tiles >= 1024)
